@@ -231,6 +231,20 @@ int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, 
     HIPCHK(hipMalloc(&ctx->tw, tw.size()));
     HIPCHK(hipMemcpyAsync(ctx->tw, tw.data(), tw.size(), hipMemcpyHostToDevice, ctx->stream));
     ctx->bytes += tw.size();
+    // band tables (kernels.hpp): a margin of rounding keeps every mode that
+    // the kernels' own test k^2 <= kM^2 could take
+    const int nh = n / 2;
+    std::vector<int> zl(2 * (nh + 1), n);
+    zl[nh] = -1;
+    for (int x = 0; x < nh; x++) {
+        const double rem = ctx->kM2 * (1 + 1e-12) - (x * dkx) * (x * dkx);
+        zl[x] = rem < 0 ? -1 : std::min(nh, int(std::sqrt(rem) / dkz * (1 + 1e-12) + 1e-9));
+        if (zl[x] >= 0) zl[nh] = x;
+    }
+    ctx->xl = zl[nh];
+    HIPCHK(hipMalloc((void**)&ctx->zl, zl.size() * sizeof(int)));
+    HIPCHK(hipMemcpyAsync(ctx->zl, zl.data(), zl.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+    ctx->bytes += zl.size() * sizeof(int);
     int r = ensure_work(ctx, 6);
     if (r) return r;
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -244,7 +258,7 @@ int bfpsh_destroy(bfpsh_ctx* ctx) {
     if (ctx->stream) {
         (void)hipSetDevice(ctx->device);
         (void)hipStreamSynchronize(ctx->stream);
-        for (void* p : {ctx->v0, ctx->v1, ctx->v2, ctx->work, ctx->ru, ctx->rgrad, ctx->tw,
+        for (void* p : {ctx->v0, ctx->v1, ctx->v2, ctx->work, ctx->ru, ctx->rgrad, ctx->tw, (void*)ctx->zl,
                         (void*)ctx->d_pos, (void*)ctx->d_rhs, (void*)ctx->d_tab, (void*)ctx->d_famp,
                         (void*)ctx->d_rank, (void*)ctx->d_samp})
             if (p && !in_slab(ctx, p)) (void)hipFree(p);
@@ -307,7 +321,10 @@ int bfpsh_put_cfield(bfpsh_ctx* ctx, int which, const void* host) {
     else host_to_planar<double>((const double*)host, (double*)tmp.data(), ctx->n);
     HIPCHK(hipMemcpyAsync(dst, tmp.data(), bytes, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (which == BFPSH_CVORTICITY) ctx->ru_valid = false;
+    if (which == BFPSH_CVORTICITY) {
+        ctx->ru_valid = false;
+        ctx->outside = 1;
+    }
     return BFPSH_OK;
 }
 
@@ -998,6 +1015,7 @@ struct bfpsh_ensemble {
     hipGraphExec_t exec = nullptr;
     bool captured_ru = false;          // the graph writes the real velocity
     std::vector<char> captured_fixed;  // per class: the graph holds the band-amplitude launches
+    std::vector<char> captured_full;   // per class: its launches move the whole half spectrum
     static constexpr int NPB = 4;      // neighbour counts batched in one step
     PartBatch pb[NPB];                 // tracer-loop groups, one per neighbour count
     int ngroups = 0;                   // groups the captured graph launches
@@ -1061,6 +1079,18 @@ static bool class_any_fixed(const bfpsh_ensemble::Cls& c) {
     return false;
 }
 
+// some box of the class may hold modes outside the dealiasing sphere
+static bool class_any_full(const bfpsh_ensemble* e, const bfpsh_ensemble::Cls& c) {
+    for (int i : c.members)
+        if (e->boxes[i]->outside) return true;
+    return false;
+}
+static bool full_changed(const bfpsh_ensemble* e) {
+    for (size_t ci = 0; ci < e->cls.size(); ci++)
+        if (ci >= e->captured_full.size() || bool(e->captured_full[ci]) != class_any_full(e, e->cls[ci])) return true;
+    return false;
+}
+
 // the captured graph no longer matches the boxes' forcing choices
 static bool fixed_changed(const bfpsh_ensemble* e) {
     if (e->captured_fixed.size() != e->cls.size()) return true;
@@ -1099,6 +1129,7 @@ static int ensemble_capture(bfpsh_ensemble* e, bool with_ru, int ngroups) {
     EHIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
     int rc = BFPSH_OK;
     e->captured_fixed.assign(e->cls.size(), 0);
+    e->captured_full.assign(e->cls.size(), 0);
     for (size_t ci = 0; ci < e->cls.size(); ci++) {
         auto& c = e->cls[ci];
         bfpsh_ctx* b0 = e->boxes[c.members[0]];
@@ -1108,6 +1139,8 @@ static int ensemble_capture(bfpsh_ensemble* e, bool with_ru, int ngroups) {
         d.spb = c.d_sp;
         d.any_fixed = class_any_fixed(c);
         e->captured_fixed[ci] = d.any_fixed;
+        d.full = class_any_full(e, c);
+        e->captured_full[ci] = char(d.full);
         d.v0 = b0->v0;
         d.v1 = b0->v1;
         d.v2 = b0->v2;
@@ -1240,9 +1273,10 @@ int bfpsh_ensemble_step(bfpsh_ensemble* e, const double* dt, int with_particles)
         if (r) return efail(e, r, pbox[0]->err);
     }
     // parameter values reach the graph through the device tables; a box
-    // switching to or from the fixed-injection forcing, or a change of the
-    // tracer launch shapes, changes its launches
-    if (!e->exec || e->captured_ru != any_part || (changed && fixed_changed(e)) ||
+    // switching to or from the fixed-injection forcing, an unprojected field
+    // put or projected, or a change of the tracer launch shapes, changes its
+    // launches
+    if (!e->exec || e->captured_ru != any_part || (changed && fixed_changed(e)) || full_changed(e) ||
         tracer_layout(e, ngroups) != e->captured_layout) {
         r = ensemble_capture(e, any_part, ngroups);
         if (r) return r;

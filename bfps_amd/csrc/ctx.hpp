@@ -44,6 +44,9 @@ struct bfpsh_ctx {
     void* ru = nullptr;            // real velocity, 3 planes [y][z][x]
     void* rgrad = nullptr;         // real gradient, 9 planes
     void* tw = nullptr;            // twiddles exp(-2 pi i t / N), N complex
+    int* zl = nullptr;             // band table of the sphere, then of the whole half spectrum (n/2 + 1 ints each)
+    int xl = 0;                    // largest kx index inside the sphere
+    int outside = 0;               // 1: v0 may hold modes outside the sphere (put, not projected since)
     double* d_famp = nullptr;      // per-stage band amplitude (fixed energy-injection forcing)
     bool ru_valid = false;
     StepParams sp{0.1, 0.0, 1.0, 2.0, 4.0, 1, 1};
@@ -207,6 +210,7 @@ struct BatchDesc {
     size_t bstride;
     const StepParams* spb;  // per-box parameters (device)
     bool any_fixed;
+    int full;               // 1: some box's v0 may hold modes outside the sphere
     void *v0, *v1, *v2, *w, *ru;
 };
 

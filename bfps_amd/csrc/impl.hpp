@@ -11,7 +11,7 @@
 template <typename T, int N>
 struct Impl {
     using CF = Cfg<T, N>;
-    static constexpr int B = CF::B, NT = CF::NT_PASS, NXH = CF::NXH;
+    static constexpr int NXH = CF::NXH;
     typedef C2<T> CT;
 
     // A batch of equal boxes (same N, precision, dk, dealiasing) whose
@@ -27,15 +27,18 @@ struct Impl {
         double* famp = nullptr;           // single box: its 3 band amplitudes
         StepParams sp;
         Geom g;
+        const int* zl = nullptr;          // band table of the step's passes (kernels.hpp)
+        int full = 0;                     // 1: some v0 may hold modes outside the sphere
     };
     // ---------------------------------------------------------- strided passes
     // compiled tile shapes of k_pass for this (T, N); ctx->pass_var[kind]
     // selects one per pass kind
     static constexpr PassShapes SH = pass_shapes<T, N>();
-    typedef void (*PassFn)(hipStream_t, CT*, size_t, size_t, const CT*, int, size_t, int);
-    template <int SIGN, int I>
-    static void pass_launch(hipStream_t st, CT* d, size_t es, size_t os, const CT* tw, int planes, size_t bs,
-                            int nbox) {
+    // zl: band table of a z pass of the step, or null for a whole transform
+    typedef void (*PassFn)(hipStream_t, CT*, size_t, size_t, const CT*, int, size_t, int, const int*);
+    template <int SIGN, int I, bool BAND>
+    static void pass_launch_b(hipStream_t st, CT* d, size_t es, size_t os, const CT* tw, int planes, size_t bs,
+                              int nbox, const int* zl) {
         constexpr PassShape p = SH.v[I < SH.n ? I : 0];
         constexpr int nt = (N / p.e) * p.b;
         if constexpr (p.pp) {
@@ -46,15 +49,22 @@ struct Impl {
                 int dev = 0, ncu = 0, occ = 0;
                 (void)hipGetDevice(&dev);
                 (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-                (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pass_pp<T, N, SIGN, p.e, p.b>, nt, 0);
+                (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pass_pp<T, N, SIGN, p.e, p.b, BAND>, nt, 0);
                 grid = std::max(1, ncu) * std::max(1, occ);
             }
             const int ntx = NXH / p.b, nty = N, ntiles = ntx * nty * planes * nbox;
-            k_pass_pp<T, N, SIGN, p.e, p.b><<<std::min(grid, ntiles), nt, 0, st>>>(d, es, os, tw, planes, bs, ntx,
-                                                                                   nty, ntiles);
+            k_pass_pp<T, N, SIGN, p.e, p.b, BAND><<<std::min(grid, ntiles), nt, 0, st>>>(d, es, os, tw, planes, bs,
+                                                                                         zl, ntx, nty, ntiles);
         } else {
-            k_pass<T, N, SIGN, p.e, p.b><<<dim3(NXH / p.b, N, planes * nbox), nt, 0, st>>>(d, es, os, tw, planes, bs);
+            k_pass<T, N, SIGN, p.e, p.b, BAND><<<dim3(NXH / p.b, N, planes * nbox), nt, 0, st>>>(d, es, os, tw, planes,
+                                                                                                 bs, zl);
         }
+    }
+    template <int SIGN, int I>
+    static void pass_launch(hipStream_t st, CT* d, size_t es, size_t os, const CT* tw, int planes, size_t bs,
+                            int nbox, const int* zl) {
+        if (zl) pass_launch_b<SIGN, I, true>(st, d, es, os, tw, planes, bs, nbox, zl);
+        else pass_launch_b<SIGN, I, false>(st, d, es, os, tw, planes, bs, nbox, zl);
     }
     template <int SIGN, size_t... I>
     static constexpr std::array<PassFn, kMaxPassShapes> pass_table(std::index_sequence<I...>) {
@@ -76,11 +86,11 @@ struct Impl {
     }
     // one in-place strided pass of `planes` planes of each of nbox boxes
     // (bstride complex elements apart)
-    static int pass(bfpsh_ctx* ctx, int kind, CT* d, int planes, const char* name, int nbox = 1,
-                    size_t bstride = 0) {
+    static int pass(bfpsh_ctx* ctx, int kind, CT* d, int planes, const char* name, const int* zl = nullptr,
+                    int nbox = 1, size_t bstride = 0) {
         const PassFn f = pass_fn(kind, ctx->pass_var[kind]);
         LAUNCH(name, f(ctx->stream, d, pass_estride(kind), pass_ostride(kind), (const CT*)ctx->tw, planes, bstride,
-                       nbox));
+                       nbox, zl));
         return BFPSH_OK;
     }
     static PassShapes shapes() { return SH; }
@@ -92,15 +102,11 @@ struct Impl {
     // first pass and the batched forms keep the built-in shape)
     static constexpr PassShapes SH_BS = fused_shapes<T, N>(CF::E_BS, CF::B_BS);
     static constexpr PassShapes SH_Y3 = fused_shapes<T, N>(CF::E_Y3, CF::B_Y3);
-    typedef void (*BsFn)(hipStream_t, const CT*, CT*, const CT*, const Geom&, int, size_t);
+    typedef void (*BsFn)(hipStream_t, const CT*, CT*, const CT*, const int*, int, const Geom&);
     template <int I>
-    static void bs_launch(hipStream_t st, const CT* src, CT* w, const CT* tw, const Geom& g, int nbox, size_t bstride) {
+    static void bs_launch(hipStream_t st, const CT* src, CT* w, const CT* tw, const int* zl, int full, const Geom& g) {
         constexpr PassShape p = SH_BS.v[I < SH_BS.n ? I : 0];
-        constexpr int nt = (N / p.e) * p.b;
-        k_inv_z_bs<T, N, 0, true, p.e, p.b><<<dim3(1, N, nbox), nt, 0, st>>>(src, w, tw, g, 0, bstride);
-        if (NXH / p.b > 1)
-            k_inv_z_bs<T, N, 0, false, p.e, p.b><<<dim3(NXH / p.b - 1, N, nbox), nt, 0, st>>>(src, w, tw, g, 1,
-                                                                                              bstride);
+        k_bs_inv_y<T, N, 0, p.e, p.b><<<dim3(NXH / p.b, N, 1), (N / p.e) * p.b, 0, st>>>(src, w, tw, zl, full, g, 0);
     }
     template <size_t... I>
     static constexpr std::array<BsFn, kMaxPassShapes> bs_table(std::index_sequence<I...>) {
@@ -110,13 +116,14 @@ struct Impl {
         static constexpr std::array<BsFn, kMaxPassShapes> t = bs_table(std::make_index_sequence<kMaxPassShapes>{});
         return t[(v >= 0 && v < SH_BS.n) ? v : 0];
     }
-    typedef void (*Y3Fn)(hipStream_t, const CT*, const CT*, const CT*, CT*, const CT*, const Geom&, const StepParams&);
+    typedef void (*Y3Fn)(hipStream_t, CT*, const CT*, const CT*, CT*, const CT*, const int*, int, const Geom&,
+                         const StepParams&);
     template <int S, int I>
-    static void y3_launch(hipStream_t st, const CT* w, const CT* v0, const CT* vp, CT* dst, const CT* tw,
-                          const Geom& g, const StepParams& sp) {
+    static void y3_launch(hipStream_t st, CT* w, const CT* v0, const CT* vp, CT* dst, const CT* tw, const int* zl,
+                          int full, const Geom& g, const StepParams& sp) {
         constexpr PassShape p = SH_Y3.v[I < SH_Y3.n ? I : 0];
-        k_fwd_y_update<T, N, S, false, p.e, p.b><<<dim3(NXH / p.b, N, 1), (N / p.e) * p.b, 0, st>>>(
-            w, v0, vp, dst, tw, g, sp, 0, nullptr);
+        k_y_update<T, N, S, false, p.e, p.b><<<dim3(NXH / p.b, N, 1), (N / p.e) * p.b, 0, st>>>(
+            w, v0, vp, dst, tw, zl, full, g, sp, 0, nullptr);
     }
     template <int S, size_t... I>
     static constexpr std::array<Y3Fn, kMaxPassShapes> y3_table(std::index_sequence<I...>) {
@@ -175,20 +182,21 @@ struct Impl {
                 const CT* tw = (const CT*)ctx->tw;
                 // one launch of shape v: a plain pass over the scratch plane;
                 // the first pass from cvorticity into the work planes; the
-                // last pass (stage 2) from work planes 0..2 into 3..5
+                // last pass of stage 1 from the work planes into v1 (which
+                // every step writes before it reads it) and back into them
                 auto run = [&]() {
                     if (kind == BFPSH_PASS_BS) {
-                        bs_fn(v)(ctx->stream, (const CT*)ctx->v0, (CT*)ctx->work, tw, geom(ctx), 1, 0);
+                        bs_fn(v)(ctx->stream, (const CT*)ctx->v0, (CT*)ctx->work, tw, band(ctx), ctx->outside,
+                                 geom(ctx));
                     } else if (kind == BFPSH_PASS_Y3) {
                         StepParams sp = ctx->sp;
                         sp.forcing = BFPSH_FORCING_NONE;
                         sp.famp_dev = nullptr;
-                        const CT* w = (const CT*)ctx->work;
-                        y3_fn(2, v)(ctx->stream, w, (const CT*)ctx->v0, (const CT*)ctx->v0,
-                                    (CT*)ctx->work + 3 * ctx->ps, tw, geom(ctx), sp);
+                        y3_fn(1, v)(ctx->stream, (CT*)ctx->work, (const CT*)ctx->v0, (const CT*)ctx->v1,
+                                    (CT*)ctx->v1, tw, band(ctx), ctx->outside, geom(ctx), sp);
                     } else {
                         pass_fn(kind, v)(ctx->stream, static_cast<CT*>(scratch), pass_estride(kind),
-                                         pass_ostride(kind), tw, 1, 0, 1);
+                                         pass_ostride(kind), tw, 1, 0, 1, nullptr);
                     }
                 };
                 run();  // warm-up
@@ -227,6 +235,10 @@ struct Impl {
         return rc;
     }
 
+    // band table of a context's step: of the sphere, or of the whole half
+    // spectrum when v0 may hold modes outside it
+    static const int* band(const bfpsh_ctx* ctx) { return ctx->outside ? ctx->zl + NXH + 1 : ctx->zl; }
+
     static Batch single(bfpsh_ctx* ctx, double dt) {
         Batch b;
         b.v0 = (CT*)ctx->v0;
@@ -240,24 +252,32 @@ struct Impl {
         b.sp.famp_dev = ctx->d_famp;
         b.any_fixed = b.sp.forcing == BFPSH_FORCING_FIXED_ENERGY;
         b.g = geom(ctx);
+        b.zl = band(ctx);
+        b.full = ctx->outside;
         return b;
     }
 
-    // Biot-Savart + first inverse pass: kx tile 0 with the symmetrize
-    // substitution, the remaining tiles without
+    // Biot-Savart + inverse y pass (built-in shape)
     template <int MODE>
-    static int bs_pass(bfpsh_ctx* ctx, const CT* src, CT* w, const CT* tw, const Geom& g, const char* name,
+    static int bs_pass(bfpsh_ctx* ctx, const CT* src, CT* w, const int* zl, int full, const Geom& g, const char* name,
                        int nbox = 1, size_t bstride = 0) {
-        LAUNCH("inv_z_bs_t0", (k_inv_z_bs<T, N, MODE, true><<<dim3(1, N, nbox), CF::NT_BS, 0, ctx->stream>>>(
-                                  src, w, tw, g, 0, bstride)));
-        if (NXH / CF::B_BS > 1)
-            LAUNCH(name, (k_inv_z_bs<T, N, MODE, false><<<dim3(NXH / CF::B_BS - 1, N, nbox), CF::NT_BS, 0, ctx->stream>>>(
-                              src, w, tw, g, 1, bstride)));
+        LAUNCH(name, (k_bs_inv_y<T, N, MODE><<<dim3(NXH / CF::B_BS, N, nbox), CF::NT_BS, 0, ctx->stream>>>(
+                         src, w, (const CT*)ctx->tw, zl, full, g, bstride)));
         return BFPSH_OK;
     }
 
-    // RK stage s of every box of the batch; ru (box 0 address) receives the
-    // real velocity of the stage-1 source when non-null
+    // The first pass of a step, from v0 into the 6 work planes
+    static int first_pass(bfpsh_ctx* ctx, const Batch& bt) {
+        if (bt.spb) return bs_pass<0>(ctx, bt.v0, bt.w, bt.zl, bt.full, bt.g, "bs_inv_y", bt.nbox, bt.bstride);
+        LAUNCH("bs_inv_y", bs_fn(ctx->pass_var[BFPSH_PASS_BS])(ctx->stream, bt.v0, bt.w, (const CT*)ctx->tw, bt.zl,
+                                                               bt.full, bt.g));
+        return BFPSH_OK;
+    }
+
+    // RK stage s of every box of the batch, from the y-transformed velocity
+    // and vorticity in the work planes to the new stage (and, for s < 3, its
+    // y-transformed fields); ru (box 0 address) receives the real velocity of
+    // the stage-1 source when non-null
     static int stage(bfpsh_ctx* ctx, int s, const Batch& bt, T* ru) {
         const Geom& g = bt.g;
         const int nb = bt.nbox;
@@ -276,36 +296,30 @@ struct Impl {
                 LAUNCH("band_amplitude", (k_band_amplitude<T, N><<<1, 256, 0, ctx->stream>>>(
                                              src, bt.famp + (s - 1), g, bt.sp.famp, bt.sp.fk0, bt.sp.fk1, 0, nullptr, s)));
         }
-        if (bt.spb) {
-            int r = bs_pass<0>(ctx, src, w, tw, g, "inv_z_bs", nb, bs);
-            if (r) return r;
-        } else {
-            LAUNCH("inv_z_bs", bs_fn(ctx->pass_var[BFPSH_PASS_BS])(ctx->stream, src, w, tw, g, 1, 0));
-        }
         {
-            int r = pass(ctx, BFPSH_PASS_Y_INV, w, 6, "inv_y", nb, bs);
+            int r = pass(ctx, BFPSH_PASS_Z_INV, w, 6, "inv_z", bt.zl, nb, bs);
             if (r) return r;
         }
         if constexpr (RowsW<T, N>::ok && !BFPSH_ROWS_TILE)
             LAUNCH("rows_cross", (k_rows_cross_w<T, N><<<dim3(N * N / 2 / RowsW<T, N>::RPB, nb), RowsW<T, N>::NT, 0,
-                                                         ctx->stream>>>(w, ru, tw, T(double(N) * N * N), bs)));
+                                                         ctx->stream>>>(w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
         else
             LAUNCH("rows_cross", (k_rows_cross<T, N><<<dim3(N * N / 2 / CF::RP, nb), CF::NT_ROW, 0, ctx->stream>>>(
-                                      w, ru, tw, T(double(N) * N * N), bs)));
+                                      w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
         {
-            int r = pass(ctx, BFPSH_PASS_Z_FWD, w, 3, "fwd_z", nb, bs);
+            int r = pass(ctx, BFPSH_PASS_Z_FWD, w, 3, "fwd_z", bt.zl, nb, bs);
             if (r) return r;
         }
         const dim3 tiles3(NXH / CF::B_Y3, N, nb);
-        const char* nm = s == 1 ? "fwd_y_update1" : (s == 2 ? "fwd_y_update2" : "fwd_y_update3");
+        const char* nm = s == 1 ? "y_update1" : (s == 2 ? "y_update2" : "y_update3");
         const CT* vp = s == 1 ? v1 : (s == 2 ? v1 : v2);
         CT* dst = s == 1 ? v1 : (s == 2 ? v2 : v0);
         if (bt.spb) {
-            if (s == 1) LAUNCH(nm, (k_fwd_y_update<T, N, 1, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, g, bt.sp, bs, bt.spb)));
-            else if (s == 2) LAUNCH(nm, (k_fwd_y_update<T, N, 2, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, g, bt.sp, bs, bt.spb)));
-            else LAUNCH(nm, (k_fwd_y_update<T, N, 3, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, g, bt.sp, bs, bt.spb)));
+            if (s == 1) LAUNCH(nm, (k_y_update<T, N, 1, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, bt.zl, bt.full, g, bt.sp, bs, bt.spb)));
+            else if (s == 2) LAUNCH(nm, (k_y_update<T, N, 2, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, bt.zl, bt.full, g, bt.sp, bs, bt.spb)));
+            else LAUNCH(nm, (k_y_update<T, N, 3, true><<<tiles3, CF::NT_Y3, 0, ctx->stream>>>(w, v0, vp, dst, tw, bt.zl, bt.full, g, bt.sp, bs, bt.spb)));
         } else {
-            LAUNCH(nm, y3_fn(s, ctx->pass_var[BFPSH_PASS_Y3])(ctx->stream, w, v0, vp, dst, tw, g, bt.sp));
+            LAUNCH(nm, y3_fn(s, ctx->pass_var[BFPSH_PASS_Y3])(ctx->stream, w, v0, vp, dst, tw, bt.zl, bt.full, g, bt.sp));
         }
         return BFPSH_OK;
     }
@@ -320,6 +334,8 @@ struct Impl {
             ru = (T*)ctx->ru;
         }
         const Batch bt = single(ctx, dt);
+        r = first_pass(ctx, bt);
+        if (r) return r;
         r = stage(ctx, 1, bt, ru);
         if (r) return r;
         if (particles) {
@@ -350,12 +366,16 @@ struct Impl {
         bt.ru = (T*)d.ru;
         bt.sp = ctx->sp;
         bt.g = geom(ctx);
+        bt.full = d.full;
+        bt.zl = d.full ? ctx->zl + NXH + 1 : ctx->zl;
         return batch_step(ctx, bt);
     }
 
     // The field part of one step of a whole batch (the tracers of each box
     // are advanced separately with the stage-1 real velocity left in ru)
     static int batch_step(bfpsh_ctx* ctx, const Batch& bt) {
+        int r0 = first_pass(ctx, bt);
+        if (r0) return r0;
         for (int s = 1; s <= 3; s++) {
             int r = stage(ctx, s, bt, s == 1 ? bt.ru : nullptr);
             if (r) return r;
@@ -379,6 +399,7 @@ struct Impl {
         const size_t ps = size_t(N) * N * NXH;
         LAUNCH("lowpass_divfree", (k_lowpass_divfree<T><<<(ps + 255) / 256, 256, 0, ctx->stream>>>((CT*)ctx->v0, geom(ctx))));
         ctx->ru_valid = false;
+        ctx->outside = 0;
         return BFPSH_OK;
     }
 
@@ -389,11 +410,11 @@ struct Impl {
         if (r) return r;
         CT* w = (CT*)ctx->work;
         const CT* tw = (const CT*)ctx->tw;
-        r = bs_pass<1>(ctx, (const CT*)ctx->v0, w, tw, geom(ctx), "inv_z_bs_u");
+        r = bs_pass<1>(ctx, (const CT*)ctx->v0, w, ctx->zl, 0, geom(ctx), "bs_inv_y_u");
         if (r) return r;
-        r = pass(ctx, BFPSH_PASS_Y_INV, w, 3, "inv_y");
+        r = pass(ctx, BFPSH_PASS_Z_INV, w, 3, "inv_z", ctx->zl);
         if (r) return r;
-        LAUNCH("rows_c2r3", (k_rows_c2r<T, N, 3><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(w, (T*)ctx->ru, tw)));
+        LAUNCH("rows_c2r3", (k_rows_c2r<T, N, 3><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(w, (T*)ctx->ru, tw, ctx->xl)));
         ctx->ru_valid = true;
         return BFPSH_OK;
     }
@@ -405,11 +426,11 @@ struct Impl {
         if (r) return r;
         CT* w = (CT*)ctx->work;
         const CT* tw = (const CT*)ctx->tw;
-        r = bs_pass<2>(ctx, (const CT*)ctx->v0, w, tw, geom(ctx), "inv_z_bs_grad");
+        r = bs_pass<2>(ctx, (const CT*)ctx->v0, w, ctx->zl, 0, geom(ctx), "bs_inv_y_grad");
         if (r) return r;
-        r = pass(ctx, BFPSH_PASS_Y_INV, w, 9, "inv_y");
+        r = pass(ctx, BFPSH_PASS_Z_INV, w, 9, "inv_z", ctx->zl);
         if (r) return r;
-        LAUNCH("rows_c2r9", (k_rows_c2r<T, N, 9><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(w, (T*)ctx->rgrad, tw)));
+        LAUNCH("rows_c2r9", (k_rows_c2r<T, N, 9><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(w, (T*)ctx->rgrad, tw, ctx->xl)));
         return BFPSH_OK;
     }
 
@@ -423,7 +444,7 @@ struct Impl {
         if (r) return r;
         r = pass(ctx, BFPSH_PASS_Y_INV, d, NC, "field_inv_y");
         if (r) return r;
-        LAUNCH("field_rows_c2r", (k_rows_c2r<T, N, NC><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(d, (T*)d, tw)));
+        LAUNCH("field_rows_c2r", (k_rows_c2r<T, N, NC><<<N * N / 2 / CF::RP, CF::NT_ROW, 0, ctx->stream>>>(d, (T*)d, tw, N)));
         return BFPSH_OK;
     }
     template <int NC>
@@ -461,6 +482,7 @@ struct Impl {
         const size_t ps = size_t(N) * N * NXH;
         LAUNCH("curl", (k_curl<T><<<(ps + 255) / 256, 256, 0, ctx->stream>>>((const CT*)ctx->work, (CT*)ctx->v0, geom(ctx))));
         ctx->ru_valid = false;
+        ctx->outside = 0;
         return symmetrize(ctx, ctx->v0, 3);
     }
 

@@ -12,10 +12,22 @@
 // (low_pass, bfps/cpp/kspace.cpp:235-253) and the time step never writes it
 // (bfps/cpp/vorticity_equation.cpp:372), so it is identically zero.
 //
-// Inverse 3D transform = z pass (within ky slab) -> y pass -> x (c2r) pass;
-// forward = x (r2c) -> z -> y.  The real-space array therefore comes out
-// as [y][z][x]; the x passes work on pairs of rows (z, z+1) packed as the
-// real and imaginary parts of one complex sequence.
+// The step's inverse transforms run y pass -> z pass -> x (c2r) pass and its
+// forward transforms x (r2c) -> z -> y, so that the last forward pass of one
+// Runge-Kutta stage and the first inverse pass of the next are both along y
+// and run in one kernel (k_y_update).  Standalone fields run z -> y -> x and
+// x -> z -> y.  The real-space array comes out as [y][z][x]; the x passes
+// work on pairs of rows (z, z+1) packed as the real and imaginary parts of
+// one complex sequence.
+//
+// Band table.  Outside the dealiasing sphere k^2 <= kM^2 the velocity is zero
+// and so is the vorticity (unless a caller put unprojected data).  Where the
+// pencil along y at (kx, kz) lies outside the sphere altogether (21 % of the
+// pencils with the smooth filter, 65 % under the two-thirds rule) the step
+// neither transforms nor moves it: zl[kx] is the largest |kz| of column kx
+// that reaches the sphere (-1: none; not increasing with kx), zl[N / 2] the
+// largest such kx.  Every kernel of the step reads the same table, so what
+// one leaves unwritten no other reads.
 #pragma once
 #include "fft.hpp"
 
@@ -48,8 +60,8 @@ template <typename T, int N>
 struct Cfg {
     static constexpr int NXH = N / 2;
     static constexpr int RMAX = 16;  // radix cap of the LDS-tile FFT (row passes)
-    // strided passes: register-resident FFT, E complex values per thread and
-    // field (all radices divide E)
+    // plain strided passes: register-resident FFT, E complex values per
+    // thread (all radices divide E)
     static constexpr int ereg() {
         if (N % 3 == 0) return 12;
         if (N <= 16) return N;
@@ -57,7 +69,6 @@ struct Cfg {
         return 8;
     }
     static constexpr int E = ereg();
-    static constexpr int G = N / E;  // thread groups per column
     // columns per strided tile: BFPSH_TILE_BYTES-byte row segments (default
     // 128) in at most lds bytes of LDS
     static constexpr int bcap(int lds) {
@@ -74,32 +85,31 @@ struct Cfg {
     // (their three components in registers need the smaller workgroups)
     static constexpr int B = bcap(BFPSH_TILE_LDS);
     static constexpr int BF = bcap(65536);
-    static constexpr int NT = G * B;
-    // Biot-Savart pass: three source components stay in registers; half the
-    // columns (when NT would exceed 512) keep it within a 256-VGPR budget
-#ifndef BFPSH_E_BS
-#define BFPSH_E_BS 0
-#endif
-    static constexpr int E_BS = (sizeof(T) == 4 && N == 512 && BFPSH_E_BS > 0 && N % BFPSH_E_BS == 0) ? BFPSH_E_BS : E;
-    static constexpr int G_BS = N / E_BS;
-    static constexpr int B_BS = (G_BS * BF > 512 && BF > 1) ? BF / 2 : BF;
-    static constexpr int NT_BS = G_BS * B_BS;
+    // fused y passes (Biot-Savart, update): three components stay in
+    // registers.  Small boxes run one short wave of workgroups, whose time is
+    // the code each one walks through once: fewer values per thread
+    static constexpr int efused() {
+        if (N % 3 == 0) return 6;
+        if (N <= 64) return 4;
+        if (N == 128) return 8;
+        return E;
+    }
+    // half the columns when the threads would exceed 512, to keep the
+    // Biot-Savart pass within a 256-VGPR budget
+    static constexpr int E_BS = efused();
+    static constexpr int B_BS = ((N / E_BS) * BF > 512 && BF > 1) ? BF / 2 : BF;
+    static constexpr int NT_BS = (N / E_BS) * B_BS;
     // last forward pass with the update epilogue (3 components in registers)
+    static constexpr int E_Y3 = efused();
     static constexpr int B_Y3 = BF;
+    static constexpr int NT_Y3 = (N / E_Y3) * B_Y3;
     // elements per thread of the plain strided pass (measured at 512^3 FP32:
-    // 16 elements x 512 threads beat 8 x 1024) and of the last forward pass
-    // (E; the register budget of its epilogue favours more threads)
+    // 16 elements x 512 threads beat 8 x 1024)
 #ifndef BFPSH_E_PASS
 #define BFPSH_E_PASS 16
 #endif
-#ifndef BFPSH_E_Y3
-#define BFPSH_E_Y3 0
-#endif
     static constexpr int pick_e(int e, int b) { return (e > 0 && N % e == 0 && (N / e) * b <= 1024) ? e : E; }
     static constexpr int E_PASS = pick_e(sizeof(T) == 4 && N == 512 ? BFPSH_E_PASS : 0, B);
-    static constexpr int NT_PASS = (N / E_PASS) * B;
-    static constexpr int E_Y3 = pick_e(sizeof(T) == 4 && N == 512 ? BFPSH_E_Y3 : 0, B_Y3);
-    static constexpr int NT_Y3 = (N / E_Y3) * B_Y3;
     static constexpr int RP = (N * int(sizeof(C2<T>)) >= 8192) ? 1 : 2;  // row pairs per row block
     // threads of the LDS-tile row passes (1024: two blocks of 512 per CU,
     // four waves per SIMD, instead of two blocks of 256)
@@ -113,13 +123,30 @@ struct Cfg {
         return lds / (row * c) > lds / (row * (c + 1)) ? int(c) : int(c + 1);
     }
     static constexpr int LS_ROW = ls_row();
-    static_assert(NT <= 1024, "tile threads");
+    static_assert((N / E_PASS) * B <= 1024 && (N / E_Y3) * B_Y3 <= 1024, "tile threads");
 };
 
 // offsets of row (y, z), row = y N + z, of a plane: complex values of a
 // spectral row and reals of a real row (the same bytes)
 template <int N> BFPSH_DEV size_t crow(size_t row) { return (row / N) * row_stride(N) + (row % N) * (N / 2); }
 template <int N> BFPSH_DEV size_t rrow(size_t row) { return (row / N) * 2 * row_stride(N) + (row % N) * N; }
+
+// Element (row n of stride YS, column col) of a plane: byte offset in 32 bits
+// where a plane is smaller than 4 GiB, so that one register of offset serves
+// every plane from its base in scalar registers
+template <typename T, int N> BFPSH_DEV auto yoff(int n, uint32_t col) {
+    constexpr uint64_t bytes = plane_size(N) * sizeof(C2<T>);
+    if constexpr (bytes < (uint64_t(1) << 32))
+        return uint32_t(uint32_t(n) * uint32_t(row_stride(N)) + col) * uint32_t(sizeof(C2<T>));
+    else
+        return (uint64_t(n) * row_stride(N) + col) * sizeof(C2<T>);
+}
+template <typename T, class O> BFPSH_DEV C2<T>& at_off(C2<T>* p, O off) {
+    return *reinterpret_cast<C2<T>*>(reinterpret_cast<char*>(p) + off);
+}
+template <typename T, class O> BFPSH_DEV const C2<T>& at_off(const C2<T>* p, O off) {
+    return *reinterpret_cast<const C2<T>*>(reinterpret_cast<const char*>(p) + off);
+}
 
 // ------------------------------------------------------------ parameters
 struct Geom {
@@ -136,6 +163,16 @@ struct StepParams {
 };
 
 BFPSH_DEV double kwave(int i, int n, double dk) { return (i <= n / 2 ? i : i - n) * dk; }
+
+// a -= k (k . a) / k^2 (force_divfree, bfps/cpp/kspace.cpp:487-519), ik2 = 1 / k^2
+template <typename T>
+BFPSH_DEV void divfree(C2<T> (&a)[3], double kx, double ky, double kz, double ik2) {
+    const T t0 = T((kx * a[0].x + ky * a[1].x + kz * a[2].x) * ik2);
+    const T t1 = T((kx * a[0].y + ky * a[1].y + kz * a[2].y) * ik2);
+    a[0] = mk<T>(T(a[0].x - t0 * kx), T(a[0].y - t1 * kx));
+    a[1] = mk<T>(T(a[1].x - t0 * ky), T(a[1].y - t1 * ky));
+    a[2] = mk<T>(T(a[2].x - t0 * kz), T(a[2].y - t1 * kz));
+}
 
 // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).
 // Remap a 2D grid so that each XCD walks a contiguous range of logical blocks
@@ -154,41 +191,48 @@ BFPSH_DEV void xcd_tile(int& bx, int& by) {
 // MODE 1: outputs u_hat (3)                        [velocity in real space]
 // MODE 2: outputs i k_j u_hat_i (9), k^2 < kM^2    [velocity gradient]
 // u_hat = i k x omega_hat / k^2 for 0 < k^2 <= kM^2, else 0
-// (compute_velocity, bfps/cpp/vorticity_equation.cpp:206-239, with the
-// symmetrize of field.cpp:900-978 applied to its kx = 0 plane by reading the
-// conjugated mirror mode; compute_gradient, bfps/cpp/field.cpp:1077-1097).
+// (compute_velocity, bfps/cpp/vorticity_equation.cpp:206-239;
+// compute_gradient, bfps/cpp/field.cpp:1077-1097).
 template <int MODE> struct BsOut { static constexpr int NF = MODE == 0 ? 6 : (MODE == 1 ? 3 : 9); };
 
-// MIRROR: the launch covers the kx tile holding kx = 0 and applies the
-// symmetrize substitution there; the other tiles use MIRROR = false
-// (blockIdx.x offset by tile0) and carry no mirror code.
-template <typename T, int N, int MODE, bool MIRROR, int E_ = Cfg<T, N>::E_BS, int B_ = Cfg<T, N>::B_BS>
-__global__ void __launch_bounds__(((N / E_) * B_))
-k_inv_z_bs(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __restrict__ tw, Geom g, int tile0,
-           size_t bstride) {
-    using CF = Cfg<T, N>;
-    // box blockIdx.z of a batch of equal boxes bstride elements apart
-    w += blockIdx.z * bstride;
-    out += blockIdx.z * bstride;
-    constexpr int B = B_, E = E_, NT = (N / E_) * B_, NXH = CF::NXH;
-    constexpr size_t PS = plane_size(N), YS = row_stride(N);
-    constexpr int NF = BsOut<MODE>::NF;
-    using F = RegFft<T, N, B, B, NT, +1>;
-    __shared__ C2<T> lds[N * B];
-    const int tid = threadIdx.x;
-    const int b = tid % B, grp = tid / B;
-    int tile, ky;
-    xcd_tile(tile, ky);
-    const int kxi = (tile + tile0) * B + b;
-    const double kx = kxi * g.dkx, kyv = kwave(ky, N, g.dky);
-    C2<T> wr[3][E];
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        const int n = F::in_row(grp, e);
-        const size_t off = size_t(ky) * YS + size_t(n) * NXH + kxi;
-#pragma unroll
-        for (int c = 0; c < 3; c++) wr[c][e] = w[c * PS + off];
+// compute_velocity symmetrizes u_hat on the kx = 0 plane: its lower half
+// (ky > N/2, or ky = 0 and kz > N/2) becomes the conjugated mirror of the
+// upper half (field.cpp:900-978).  The c2r pass takes the real part of the
+// kx = 0 sum, to which a mode and its conjugated mirror add the same, so the
+// lower half may be left out and the upper half doubled: this factor of a
+// kx = 0 mode, with no mirror to read.
+template <typename T, int N> BFPSH_DEV T plane0_factor(int ky, int kz) {
+    if (ky > N / 2 || (ky == 0 && kz > N / 2)) return T(0);
+    if (ky == N / 2 || (ky == 0 && (kz == 0 || kz == N / 2))) return T(1);  // its own mirror, or none
+    return T(2);
+}
+
+// Velocity component cu of the mode (kx, ky, kz) with vorticity a0, a1, a2,
+// zero outside 0 < k^2 <= kM^2
+template <typename T>
+BFPSH_DEV C2<T> biot_savart(int cu, C2<T> a0, C2<T> a1, C2<T> a2, double kx, double ky, double kz, double k2,
+                            double kM2) {
+    C2<T> u = mk<T>(T(0), T(0));
+    if (k2 <= kM2 && k2 > 0) {
+        // one FP64 division per element and field, then products (within
+        // an ulp of the quotients before the rounding to T)
+        const double ik2 = 1.0 / k2;
+        if (cu == 0) u = mk<T>(T(-(ky * a2.y - kz * a1.y) * ik2), T((ky * a2.x - kz * a1.x) * ik2));
+        if (cu == 1) u = mk<T>(T(-(kz * a0.y - kx * a2.y) * ik2), T((kz * a0.x - kx * a2.x) * ik2));
+        if (cu == 2) u = mk<T>(T(-(kx * a1.y - ky * a0.y) * ik2), T((kx * a1.x - ky * a0.x) * ik2));
     }
+    return u;
+}
+
+// Fields of the column (kxi, kz) from its vorticity wr (element e at row
+// F::in_row(grp, e)), inverse-transformed along y into o + f PS, f < NF.
+template <typename T, int N, int MODE, class F, int E>
+BFPSH_DEV void bs_inverse_y(C2<T> (&wr)[3][E], C2<T>* lds, const C2<T>* __restrict__ tw, C2<T>* o, int grp, int b,
+                            int kxi, int kz, const Geom& g) {
+    constexpr size_t PS = plane_size(N);
+    const uint32_t col = uint32_t(kz) * uint32_t(N / 2) + uint32_t(kxi);
+    constexpr int NF = BsOut<MODE>::NF;
+    const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
     // Velocity-type fields in a runtime loop (register arrays indexed by
     // constants only), then the vorticity copies (MODE 0) as straight-line
     // code: a runtime select between wr[0..2] would turn into a pointer into
@@ -210,48 +254,72 @@ k_inv_z_bs(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int n = F::in_row(gq, e);
-            const double kz = kwave(n, N, g.dkz);
-            const double k2 = kx * kx + kyv * kyv + kz * kz;
+            const double kyv = kwave(n, N, g.dky);
+            const double k2 = kx * kx + kyv * kyv + kzv * kzv;
             const int cu = MODE == 2 ? f % 3 : f;
-            C2<T> a0 = wr[0][e], a1 = wr[1][e], a2 = wr[2][e];
-            // symmetrized kx = 0 plane: the lower half takes conj(mirror)
-            if (MIRROR && kxi == 0 && ((ky > N / 2) || (ky == 0 && n > N / 2))) {
-                const size_t moff = size_t((N - ky) % N) * YS + size_t((N - n) % N) * NXH;
-                a0 = cconj<T>(w[moff]);
-                a1 = cconj<T>(w[PS + moff]);
-                a2 = cconj<T>(w[2 * PS + moff]);
-            }
-            C2<T> u = mk<T>(T(0), T(0));
-            if (k2 <= g.kM2 && k2 > 0) {
-                // one FP64 division per element and field, then products
-                // (within an ulp of the quotients before the rounding to T)
-                const double ik2 = 1.0 / k2;
-                if (cu == 0) u = mk<T>(T(-(kyv * a2.y - kz * a1.y) * ik2), T((kyv * a2.x - kz * a1.x) * ik2));
-                if (cu == 1) u = mk<T>(T(-(kz * a0.y - kx * a2.y) * ik2), T((kz * a0.x - kx * a2.x) * ik2));
-                if (cu == 2) u = mk<T>(T(-(kx * a1.y - kyv * a0.y) * ik2), T((kx * a1.x - kyv * a0.x) * ik2));
+            C2<T> u = biot_savart<T>(cu, wr[0][e], wr[1][e], wr[2][e], kx, kyv, kzv, k2, g.kM2);
+            if (kxi == 0) {
+                const T s = plane0_factor<T, N>(n, kz);
+                u = mk<T>(u.x * s, u.y * s);
             }
             if (MODE == 2) {
                 const int j = f / 3;
-                const double kj = j == 0 ? kx : (j == 1 ? kyv : kz);
+                const double kj = j == 0 ? kx : (j == 1 ? kyv : kzv);
                 v[e] = k2 < g.kM2 ? mk<T>(T(-kj * u.y), T(kj * u.x)) : mk<T>(T(0), T(0));
             } else {
                 v[e] = u;
             }
         }
         F::run(v, lds, tw, gq, b);
-        C2<T>* o = out + size_t(f) * PS;
+        C2<T>* of = o + size_t(f) * PS;
 #pragma unroll
-        for (int e = 0; e < E; e++) o[size_t(ky) * YS + size_t(F::out_row(gq, e)) * NXH + kxi] = v[e];
+        for (int e = 0; e < E; e++) at_off<T>(of, yoff<T, N>(F::out_row(gq, e), col)) = v[e];
     }
     if constexpr (MODE == 0) {
         sfor<0, 3>([&](auto cc) {
             constexpr int c = cc;
-            F::run(wr[c], lds, tw, grp, b);
-            C2<T>* o = out + size_t(3 + c) * PS;
+            int gq = grp, t0 = 0;
+            asm volatile("" : "+v"(gq), "+s"(t0));
+            F::run(wr[c], lds, tw + t0, gq, b);
+            C2<T>* of = o + size_t(3 + c) * PS;
 #pragma unroll
-            for (int e = 0; e < E; e++) o[size_t(ky) * YS + size_t(F::out_row(grp, e)) * NXH + kxi] = wr[c][e];
+            for (int e = 0; e < E; e++) at_off<T>(of, yoff<T, N>(F::out_row(gq, e), col)) = wr[c][e];
         });
     }
+}
+
+// Biot-Savart and the inverse y pass from the vorticity w; `full`: w may hold
+// modes outside the sphere, which the vorticity copies then keep.
+template <typename T, int N, int MODE, int E_ = Cfg<T, N>::E_BS, int B_ = Cfg<T, N>::B_BS>
+__global__ void __launch_bounds__(((N / E_) * B_))
+k_bs_inv_y(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __restrict__ tw,
+           const int* __restrict__ zl, int full, Geom g, size_t bstride) {
+    using CF = Cfg<T, N>;
+    // box blockIdx.z of a batch of equal boxes bstride elements apart
+    w += blockIdx.z * bstride;
+    out += blockIdx.z * bstride;
+    constexpr int B = B_, E = E_, NT = (N / E_) * B_, NXH = CF::NXH;
+    constexpr size_t PS = plane_size(N);
+    using F = RegFft<T, N, B, B, NT, +1>;
+    __shared__ C2<T> lds[N * B];
+    const int tid = threadIdx.x;
+    const int b = tid % B, grp = tid / B;
+    int tile, kz;
+    xcd_tile(tile, kz);
+    if (min(kz, N - kz) > zl[tile * B]) return;  // uniform: the whole tile lies outside the sphere
+    const int kxi = tile * B + b;
+    const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
+    const uint32_t col = uint32_t(kz) * uint32_t(NXH) + uint32_t(kxi);
+    C2<T> wr[3][E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = F::in_row(grp, e);
+        const double kyv = kwave(n, N, g.dky);
+        const bool in = full || kx * kx + kyv * kyv + kzv * kzv <= g.kM2;
+#pragma unroll
+        for (int c = 0; c < 3; c++) wr[c][e] = in ? at_off<T>(w + c * PS, yoff<T, N>(n, col)) : mk<T>(T(0), T(0));
+    }
+    bs_inverse_y<T, N, MODE, F, E>(wr, lds, tw, out, grp, b, kxi, kz, g);
 }
 
 // ------------------------------------------------------------ generic strided pass (in place)
@@ -261,10 +329,15 @@ k_inv_z_bs(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __
 // Tile shape: B columns, E complex values per thread (N / E threads per
 // column); the shapes a context may use are listed by pass_shapes() and
 // picked by the pass autotuner.
-template <typename T, int N, int SIGN, int E, int B>
+// BAND: the z pass of the step, which moves the rows within the band table zl
+// only: the inverse pass takes the rows beyond as zero, the forward pass does
+// not store them, and columns with no row in the band are left alone.
+template <int N> BFPSH_DEV bool in_band(int n, int lim) { return min(n, N - n) <= lim; }
+
+template <typename T, int N, int SIGN, int E, int B, bool BAND>
 __global__ void __launch_bounds__((N / E) * B)
 k_pass(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __restrict__ tw, int planes,
-       size_t bstride) {
+       size_t bstride, const int* __restrict__ zl) {
     constexpr int NT = (N / E) * B;
     using F = RegFft<T, N, B, B, NT, SIGN>;
     static_assert(F::E == E, "tile shape");
@@ -272,15 +345,32 @@ k_pass(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __
     __shared__ C2<T> lds[N * B];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
+    int lim = N;
+    if constexpr (BAND) {
+        if (zl[blockIdx.x * B] < 0) return;  // uniform
+        lim = zl[blockIdx.x * B + b];
+    }
     // blockIdx.z = box * planes + plane (boxes bstride elements apart)
     const int box = blockIdx.z / planes, plane = blockIdx.z % planes;
     C2<T>* base = data + box * bstride + plane * PS + blockIdx.y * ostride + blockIdx.x * B + b;
     C2<T> v[E];
 #pragma unroll
-    for (int e = 0; e < E; e++) v[e] = base[F::in_row(grp, e) * estride];
+    for (int e = 0; e < E; e++) {
+        const int n = F::in_row(grp, e);
+        if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? base[n * estride] : mk<T>(T(0), T(0));
+        else v[e] = base[n * estride];
+    }
     F::run(v, lds, tw, grp, b);
+    if constexpr (BAND && SIGN < 0) {
+        // (not to be sunk into the conditional stores)
 #pragma unroll
-    for (int e = 0; e < E; e++) base[F::out_row(grp, e) * estride] = v[e];
+        for (int e = 0; e < E; e++) asm volatile("" : "+v"(v[e].x), "+v"(v[e].y));
+    }
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const int n = F::out_row(grp, e);
+        if (!(BAND && SIGN < 0) || in_band<N>(n, lim)) base[n * estride] = v[e];
+    }
 }
 
 // Persistent form of k_pass: gridDim.x workgroups (as many as fit on the
@@ -289,10 +379,10 @@ k_pass(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __
 // next tile while the current one is transformed and stored, so that
 // global-memory latency hides behind the FFT (the barriers of the FFT
 // order LDS only and leave those loads in flight).
-template <typename T, int N, int SIGN, int E, int B>
+template <typename T, int N, int SIGN, int E, int B, bool BAND>
 __global__ void __launch_bounds__((N / E) * B)
 k_pass_pp(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __restrict__ tw, int planes,
-          size_t bstride, int ntx, int nty, int ntiles) {
+          size_t bstride, const int* __restrict__ zl, int ntx, int nty, int ntiles) {
     constexpr int NT = (N / E) * B;
     using F = RegFft<T, N, B, B, NT, SIGN>;
     static_assert(F::E == E, "tile shape");
@@ -300,37 +390,47 @@ k_pass_pp(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>*
     __shared__ C2<T> lds[N * B];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
-    auto base_of = [&](int t) {
+    // tile t: its column's address and (BAND) band limit
+    auto base_of = [&](int t, int& lim) {
         const int x = t % ntx, r = t / ntx, y = r % nty, zp = r / nty;
         const int box = zp / planes, plane = zp % planes;
+        lim = BAND ? zl[x * B + b] : N;
         return data + box * bstride + plane * PS + size_t(y) * ostride + size_t(x) * B + b;
+    };
+    auto load = [&](const C2<T>* p, int lim, C2<T> (&v)[E]) {
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int n = F::in_row(grp, e);
+            if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? p[n * estride] : mk<T>(T(0), T(0));
+            else v[e] = p[n * estride];
+        }
     };
     int t = blockIdx.x;
     if (t >= ntiles) return;
+    int lim, nlim = 0;
+    C2<T>* p = base_of(t, lim);
+    C2<T>* pn = nullptr;
     C2<T> cur[E], nxt[E];
-    {
-        const C2<T>* p = base_of(t);
-#pragma unroll
-        for (int e = 0; e < E; e++) cur[e] = p[F::in_row(grp, e) * estride];
-    }
+    load(p, lim, cur);
     for (;;) {
         const int tn = t + int(gridDim.x);
         const bool more = tn < ntiles;  // uniform
         if (more) {
-            const C2<T>* p = base_of(tn);
-#pragma unroll
-            for (int e = 0; e < E; e++) nxt[e] = p[F::in_row(grp, e) * estride];
+            pn = base_of(tn, nlim);
+            load(pn, nlim, nxt);
         }
         F::run(cur, lds, tw, grp, b);
-        {
-            C2<T>* p = base_of(t);
 #pragma unroll
-            for (int e = 0; e < E; e++) p[F::out_row(grp, e) * estride] = cur[e];
+        for (int e = 0; e < E; e++) {
+            const int n = F::out_row(grp, e);
+            if (!BAND || (SIGN > 0 ? lim >= 0 : in_band<N>(n, lim))) p[n * estride] = cur[e];
         }
         if (!more) break;
 #pragma unroll
         for (int e = 0; e < E; e++) cur[e] = nxt[e];
         t = tn;
+        p = pn;
+        lim = nlim;
     }
 }
 
@@ -381,7 +481,7 @@ constexpr PassShapes pass_shapes() {
     return s;
 }
 
-// Tile shapes of the fused first (Biot-Savart + inverse z) and last
+// Tile shapes of the fused first (Biot-Savart + inverse y) and last
 // (forward y + update) passes, which hold three components in registers:
 // the built-in choice first, then for N >= 512 the shapes with E in
 // {8, 16}, 64..1024 threads, at least 64-byte row segments, at most 128 KB
@@ -421,9 +521,10 @@ constexpr PassShapes fused_shapes(int e0, int b0) {
 // B[k] = (Z[k] - conj Z[N-k]) / (2 i).
 // NCOL columns at once: all global loads of a thread are issued before its
 // LDS stores.  Column col reads rows ra(col), rb(col) = base + off[col].
+// Modes k > xl lie outside the dealiasing sphere: taken as zero, not read.
 template <typename T, int N, int LS, int NCOL, int NT>
 BFPSH_DEV void rows_unpack_inverse(C2<T>* lds, const C2<T>* const (&ra)[NCOL], const C2<T>* const (&rb)[NCOL],
-                                   int tid) {
+                                   int xl, int tid) {
     constexpr int H = N / 2;
     constexpr int PER = (H + NT - 1) / NT;
 #pragma unroll
@@ -433,8 +534,8 @@ BFPSH_DEV void rows_unpack_inverse(C2<T>* lds, const C2<T>* const (&ra)[NCOL], c
         C2<T> A[NCOL], Bv[NCOL];
 #pragma unroll
         for (int col = 0; col < NCOL; col++) {
-            A[col] = ra[col][k];
-            Bv[col] = rb[col][k];
+            A[col] = k <= xl ? ra[col][k] : mk<T>(T(0), T(0));
+            Bv[col] = k <= xl ? rb[col][k] : mk<T>(T(0), T(0));
         }
 #pragma unroll
         for (int col = 0; col < NCOL; col++) {
@@ -449,9 +550,9 @@ BFPSH_DEV void rows_unpack_inverse(C2<T>* lds, const C2<T>* const (&ra)[NCOL], c
     }
 }
 template <typename T, int N, int LS>
-BFPSH_DEV void rows_pack_forward(const C2<T>* lds, int col, C2<T>* ra, C2<T>* rb, int tid, int nt) {
+BFPSH_DEV void rows_pack_forward(const C2<T>* lds, int col, C2<T>* ra, C2<T>* rb, int xl, int tid, int nt) {
     constexpr int H = N / 2;
-    for (int k = tid; k < H; k += nt) {
+    for (int k = tid; k < min(H, xl + 1); k += nt) {
         const C2<T> Z = lds[k * LS + col];
         const C2<T> M = lds[((N - k) % N) * LS + col];
         ra[k] = mk<T>(T(0.5) * (Z.x + M.x), T(0.5) * (Z.y - M.y));
@@ -466,7 +567,8 @@ BFPSH_DEV void rows_pack_forward(const C2<T>* lds, int col, C2<T>* ra, C2<T>* rb
 //      velocity ru (3 real planes [y][z][x]) for the tracers.
 template <typename T, int N>
 __global__ void __launch_bounds__((Cfg<T, N>::NT_ROW))
-k_rows_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restrict__ tw, T npoints, size_t bstride) {
+k_rows_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restrict__ tw, const int* __restrict__ zl,
+             T npoints, size_t bstride) {
     using CF = Cfg<T, N>;
     // LDS row stride: odd, so lanes striding by rows hit distinct banks
     constexpr int RP = CF::RP, NT = CF::NT_ROW, NXH = CF::NXH, LS = CF::LS_ROW;
@@ -478,6 +580,7 @@ k_rows_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restri
     // the 1/npoints normalization as a product (exact for the power-of-two
     // sizes, within an ulp of the quotient otherwise)
     const T inp = T(1) / npoints;
+    const int xl = zl[NXH];
     const int tid = threadIdx.x;
     const int q0 = blockIdx.x * RP;  // first row pair; rows (y, z) flattened: row = y*N + z
     {
@@ -491,7 +594,7 @@ k_rows_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restri
                 ra[c * RP + p] = data + c * PS + crow<N>(row);
                 rb[c * RP + p] = data + c * PS + crow<N>(row) + NXH;
             }
-        rows_unpack_inverse<T, N, LS, 6 * RP, NT>(lds, ra, rb, tid);
+        rows_unpack_inverse<T, N, LS, 6 * RP, NT>(lds, ra, rb, xl, tid);
     }
     __syncthreads();
     fft_tile<T, N, 6 * RP, LS, NT, CF::RMAX, +1>(lds, tw, tid);
@@ -525,7 +628,7 @@ k_rows_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restri
         for (int p = 0; p < RP; p++) {
             const size_t row = size_t(q0 + p) * 2;
             rows_pack_forward<T, N, LS>(lds, c * RP + p, data + c * PS + crow<N>(row),
-                                        data + c * PS + crow<N>(row) + NXH, tid, NT);
+                                        data + c * PS + crow<N>(row) + NXH, xl, tid, NT);
         }
 }
 
@@ -574,10 +677,12 @@ template <typename T, int N, int SIGN, int NCG>
 BFPSH_DEV void rows_w_fft(C2<T> (&v)[NCG][8], C2<T>* reg, const C2<T>* __restrict__ tw, int g) {
     using RW = RowsW<T, N>;
     using F = RegFft<T, N, 1, 1, RW::G, SIGN>;
-    // an opaque copy of the twiddle pointer: the twiddles are re-read (from
-    // cache) per group instead of being held in registers across all of them
-    const C2<T>* twl = tw;
-    asm volatile("" : "+s"(twl));
+    // an opaque twiddle offset: the twiddles are re-read (from cache) per
+    // group instead of being held in registers across all of them (an opaque
+    // pointer would lose its address space and be read by flat loads)
+    int t0 = 0;
+    asm volatile("" : "+s"(t0));
+    const C2<T>* twl = tw + t0;
     // likewise the LDS slot addresses are recomputed per group
     int gl = g;
     asm volatile("" : "+v"(gl));
@@ -606,8 +711,8 @@ BFPSH_DEV C2<T> shfl2(C2<T> a, int src) {
 
 template <typename T, int N>
 __global__ void __launch_bounds__(256, BFPSH_RW_WAVES)
-k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restrict__ tw, T npoints,
-               size_t bstride) {
+k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restrict__ tw,
+               const int* __restrict__ zl, T npoints, size_t bstride) {
     using RW = RowsW<T, N>;
     constexpr int E = RW::E, G = RW::G, H = RW::H, RPB = RW::RPB, NXH = N / 2;
     constexpr size_t PS = plane_size(N), YS = row_stride(N);
@@ -616,6 +721,7 @@ k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __rest
     data += blockIdx.y * bstride;
     if (ru) ru += blockIdx.y * 2 * bstride;
     const T inp = T(1) / npoints;  // normalization as a product, as k_rows_cross
+    const int xl = zl[NXH];  // modes beyond are zero: neither read nor written
     const int tid = threadIdx.x;
     const int rp = tid / G, g = tid % G;
     const int partner = (tid & 63) - g + (G - g) % G;  // lane holding index N - k
@@ -632,8 +738,9 @@ k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __rest
         for (int c = 0; c < 3; c++)
 #pragma unroll
             for (int m = 0; m < H; m++) {
-                A[c][m] = data[(c0 + c) * PS + ra + g + G * m];
-                B[c][m] = data[(c0 + c) * PS + rb + g + G * m];
+                const bool in = g + G * m <= xl;
+                A[c][m] = in ? data[(c0 + c) * PS + ra + g + G * m] : mk<T>(T(0), T(0));
+                B[c][m] = in ? data[(c0 + c) * PS + rb + g + G * m] : mk<T>(T(0), T(0));
             }
     };
     auto unpack = [&](C2<T> (&vv)[3][E]) {
@@ -706,6 +813,7 @@ k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __rest
             const C2<T> Z = f[c][RW::tau_inv(m)];
             C2<T> M = shfl2<T>(f[c][RW::tau_inv(E - 1 - m)], partner);
             if (g == 0) M = f[c][RW::tau_inv((E - m) % E)];
+            if (g + G * m > xl) continue;
             data[c * PS + ra + g + G * m] = mk<T>(T(0.5) * (Z.x + M.x), T(0.5) * (Z.y - M.y));
             data[c * PS + rb + g + G * m] = mk<T>(T(0.5) * (Z.y + M.y), T(-0.5) * (Z.x - M.x));
         }
@@ -718,7 +826,7 @@ k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __rest
 // of its rows before writing them).
 template <typename T, int N, int NC>
 __global__ void __launch_bounds__((Cfg<T, N>::NT_ROW))
-k_rows_c2r(const C2<T>* data, T* out, const C2<T>* __restrict__ tw) {
+k_rows_c2r(const C2<T>* data, T* out, const C2<T>* __restrict__ tw, int xl) {
     using CF = Cfg<T, N>;
     constexpr int NG = NC < 3 ? NC : 3;
     constexpr int RP = CF::RP, NT = CF::NT_ROW, NXH = CF::NXH, LS = NG * RP + 1;
@@ -739,7 +847,7 @@ k_rows_c2r(const C2<T>* data, T* out, const C2<T>* __restrict__ tw) {
                     ra[c * RP + p] = data + (c0 + c) * PS + crow<N>(row);
                     rb[c * RP + p] = data + (c0 + c) * PS + crow<N>(row) + NXH;
                 }
-            rows_unpack_inverse<T, N, LS, NG * RP, NT>(lds, ra, rb, tid);
+            rows_unpack_inverse<T, N, LS, NG * RP, NT>(lds, ra, rb, xl, tid);
         }
         __syncthreads();
         fft_tile<T, N, NG * RP, LS, NT, CF::RMAX, +1>(lds, tw, tid);
@@ -782,7 +890,7 @@ k_rows_r2c(const T* data, C2<T>* out, const C2<T>* __restrict__ tw) {
             for (int p = 0; p < RP; p++) {
                 const size_t row = size_t(q0 + p) * 2;
                 rows_pack_forward<T, N, LS>(lds, c * RP + p, out + (c0 + c) * PS + crow<N>(row),
-                                            out + (c0 + c) * PS + crow<N>(row) + NXH, tid, NT);
+                                            out + (c0 + c) * PS + crow<N>(row) + NXH, N, tid, NT);
             }
         __syncthreads();
     }
@@ -793,153 +901,211 @@ k_rows_r2c(const T* data, C2<T>* out, const C2<T>* __restrict__ tw) {
 // (vorticity_equation::step, bfps/cpp/vorticity_equation.cpp:358-439), fused
 // with the tail of omega_nonlin (:323-355): dealias (kspace.cpp:461-485),
 // curl, forcing (:241-288), force_divfree (kspace.cpp:487-519).
-// data: planes 0..2 hold the output of the z forward pass ([y][kz][kx]).
+// w: planes 0..2 hold the output of the z forward pass ([y][kz][kx]).
 // v0 = omega(t); vp = previous stage (stage 2: v1, stage 3: v2); dst receives
 // the new stage (stage 3 writes v0 in place and applies the final projection).
+// Stages 1 and 2 go on with the first pass of the next stage while its
+// vorticity is in registers: Biot-Savart and the inverse y pass into planes
+// 0..5 of w (a workgroup reads its columns before it writes them).  That
+// saves reading the new vorticity back (3 N^3) and one launch a stage.
+//
+// Outside the sphere the stages are zero and stay unwritten (v1 and v2 start
+// as zeros); stage 3 keeps v0 there, projected, when `full` says that it may
+// hold something.  The integrating factor exp(-nu k^2 dt c) is combined from
+// one value per ky, in an LDS table, and one per thread for its (kx, kz),
+// instead of one exponential per mode (two in stage 2): from
+// e = exp - 1 as 1 + (a + b + a b), whose error is that of its last rounding
+// like the exponential's own, while the factors stay above exp(-1/2); the
+// product of exponentials where viscosity damps the last modes faster.
 template <typename T, int N, int STAGE, bool BATCH, int E_ = Cfg<T, N>::E_Y3, int B_ = Cfg<T, N>::B_Y3>
 __global__ void __launch_bounds__(((N / E_) * B_))
-k_fwd_y_update(const C2<T>* __restrict__ data, const C2<T>* v0, const C2<T>* __restrict__ vp,
-               C2<T>* dst, const C2<T>* __restrict__ tw, Geom g, StepParams sp0, size_t bstride,
-               const StepParams* __restrict__ spb) {
+k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* __restrict__ tw,
+           const int* __restrict__ zl, int full, Geom g, StepParams sp0, size_t bstride,
+           const StepParams* __restrict__ spb) {
     using CF = Cfg<T, N>;
     // BATCH: box blockIdx.z of a batch, its fields bstride elements apart and
     // its own physics parameters in spb (a separate instantiation keeps the
     // single-box kernel's registers free of the batch bookkeeping)
     if constexpr (BATCH) {
-        data += blockIdx.z * bstride;
+        w += blockIdx.z * bstride;
         v0 += blockIdx.z * bstride;
         vp += blockIdx.z * bstride;
         dst += blockIdx.z * bstride;
     }
     const StepParams sp = BATCH ? spb[blockIdx.z] : sp0;
     constexpr int B = B_, E = E_, NT = (N / E_) * B_, NXH = CF::NXH;
-    constexpr size_t PS = plane_size(N), YS = row_stride(N);
+    constexpr size_t PS = plane_size(N);
     using F = RegFft<T, N, B, B, NT, -1>;
     __shared__ C2<T> lds[N * B];
+    __shared__ double ify[STAGE == 2 ? 2 : 1][N];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
     // tiles narrower than a 128-byte line (1024^3): neighbouring tiles, the
     // two halves of each line, run on the same XCD and share its L2
     int tile = blockIdx.x, kz = blockIdx.y;
     if constexpr (B * sizeof(C2<T>) < 128) xcd_tile(tile, kz);
+    const int kza = min(kz, N - kz);
+    if (kza > zl[tile * B]) return;  // uniform: the whole tile lies outside the sphere
     const int kxi = tile * B + b;
+    const bool col_in = kza <= zl[kxi];
+    const uint32_t col = uint32_t(kz) * uint32_t(NXH) + uint32_t(kxi);
     C2<T> res[3][E];
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        const C2<T>* src = data + c * PS + size_t(kz) * NXH + kxi;
+    for (int c = 0; c < 3; c++)
 #pragma unroll
-        for (int e = 0; e < E; e++) res[c][e] = src[size_t(F::in_row(grp, e)) * YS];
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) F::run(res[c], lds, tw, grp, b);
+        for (int e = 0; e < E; e++)
+            res[c][e] = col_in ? at_off<T>(w + c * PS, yoff<T, N>(F::in_row(grp, e), col)) : mk<T>(T(0), T(0));
     const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
-    const double ikM2 = 1.0 / g.kM2;
+    const double dt = sp.dt, nud = sp.nu * dt * (STAGE == 1 ? 1.0 : 0.5);
+    const bool slow = fabs(nud) * g.kM2 < 0.5;  // uniform
+    auto if_part = [&](double x) { return slow ? expm1(x) : exp(x); };
+    auto if_of = [&](double p, double q) { return slow ? 1.0 + fma(p, q, p + q) : p * q; };
+    for (int i = tid; i < N; i += NT) {
+        const double k = kwave(i, N, g.dky);
+        ify[0][i] = if_part(-nud * k * k);
+        if constexpr (STAGE == 2) ify[1][i] = if_part(nud * k * k);
+    }
+    const double ifxz = if_part(-nud * (kx * kx + kzv * kzv));
+    const double ifxz1 = STAGE == 2 ? if_part(nud * (kx * kx + kzv * kzv)) : 0.0;
+    __syncthreads();
+    // one component after the other; an opaque group index and table offset
+    // per component, so that twiddles and LDS addresses are not held across,
+    // and opaque results, so that the last butterflies are not sunk into the
+    // conditional code below (which would keep all their inputs alive)
 #pragma unroll
-    for (int i = 0; i < E; i++) {
-        const int ky = F::out_row(grp, i);
+    for (int c = 0; c < 3; c++) {
+        int gq = grp, t0 = 0;
+        asm volatile("" : "+v"(gq), "+s"(t0));
+        F::run(res[c], lds, tw + t0, gq, b);
+#pragma unroll
+        for (int e = 0; e < E; e++) asm volatile("" : "+v"(res[c][e].x), "+v"(res[c][e].y));
+    }
+    const double ikM2 = 1.0 / g.kM2;
+    const double fk1sq = sp.fk1 * sp.fk1 * (1 + 1e-12);
+    // v0 and vp of element i + 1 are requested before element i is computed
+    // (few waves fit beside the three components, so their loads must not
+    // wait for one another); nothing else of an element is kept across
+    C2<T> p0[2][3], p1[2][3];
+    auto fetch = [&](int i, C2<T> (&q0)[3], C2<T> (&q1)[3]) {
+        int gq = grp;
+        asm volatile("" : "+v"(gq));
+        const int ky = F::out_row(gq, i);
+        const double kyv = kwave(ky, N, g.dky);
+        if (kx * kx + kyv * kyv + kzv * kzv <= g.kM2 || (STAGE == 3 && full)) {
+            const auto off = yoff<T, N>(ky, col);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                q0[c] = at_off<T>(v0 + c * PS, off);
+                if (STAGE > 1) q1[c] = at_off<T>(vp + c * PS, off);
+            }
+        }
+    };
+    fetch(0, p0[0], p1[0]);
+    sfor<0, E>([&](auto ii) {
+        constexpr int i = ii;
+        if constexpr (i + 1 < E) fetch(i + 1, p0[(i + 1) % 2], p1[(i + 1) % 2]);
+        const C2<T>(&w0)[3] = p0[i % 2];
+        const C2<T>(&w1)[3] = p1[i % 2];
+        int gq = grp;
+        asm volatile("" : "+v"(gq));
+        const int ky = F::out_row(gq, i);
         const double kyv = kwave(ky, N, g.dky);
         const double k2 = kx * kx + kyv * kyv + kzv * kzv;
-        const size_t off = size_t(ky) * YS + size_t(kz) * NXH + kxi;
-        // dealias
-        C2<T> a[3];
-        if (g.smooth) {
-            const double r = k2 * ikM2;
-            const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4, r16 = r8 * r8;
-            const double flt = exp(-36.0 * (r16 * r2));
+        const auto off = yoff<T, N>(ky, col);
+        C2<T> nv[3];
+        bool write = true;
+        if (k2 <= g.kM2) {
+            // dealias
+            C2<T> a[3];
+            if (g.smooth) {
+                const double r = k2 * ikM2;
+                const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4, r16 = r8 * r8;
+                const double flt = exp(-36.0 * (r16 * r2));
 #pragma unroll
-            for (int c = 0; c < 3; c++) a[c] = mk<T>(T(res[c][i].x * flt), T(res[c][i].y * flt));
-        } else {
-#pragma unroll
-            for (int c = 0; c < 3; c++) a[c] = k2 >= g.kM2 ? mk<T>(T(0), T(0)) : res[c][i];
-        }
-        // curl: i k x a
-        C2<T> cu[3];
-        cu[0] = mk<T>(T(-(kyv * a[2].y - kzv * a[1].y)), T(kyv * a[2].x - kzv * a[1].x));
-        cu[1] = mk<T>(T(-(kzv * a[0].y - kx * a[2].y)), T(kzv * a[0].x - kx * a[2].x));
-        cu[2] = mk<T>(T(-(kx * a[1].y - kyv * a[0].y)), T(kx * a[1].x - kyv * a[0].x));
-        // forcing with the stage's source vorticity
-        const C2<T>* srcv = STAGE == 1 ? v0 : vp;
-        if (sp.forcing == 1 || sp.forcing == 3) {
-            const double kn = sqrt(k2);
-            if (sp.fk0 <= kn && sp.fk1 >= kn) {
-                const double amp = sp.forcing == 1 ? sp.famp : sp.famp_dev[STAGE - 1];
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const C2<T> s = srcv[c * PS + off];
-                    cu[c] = mk<T>(T(cu[c].x + amp * double(s.x) * 1.0), T(cu[c].y + amp * double(s.y) * 1.0));
-                }
-            }
-        } else if (sp.forcing == 2) {
-            if (kxi == 0 && kz == 0 && (ky == sp.fmode || ky == N - sp.fmode))
-                cu[2].x = T(cu[2].x - sp.famp * 1.0 / 2);
-        }
-        // force_divfree
-        if (k2 > 0) {
-            const double ik2 = 1.0 / k2;  // one division, then products
-            const T t0 = T((kx * cu[0].x + kyv * cu[1].x + kzv * cu[2].x) * ik2);
-            const T t1 = T((kx * cu[0].y + kyv * cu[1].y + kzv * cu[2].y) * ik2);
-            cu[0] = mk<T>(T(cu[0].x - t0 * kx), T(cu[0].y - t1 * kx));
-            cu[1] = mk<T>(T(cu[1].x - t0 * kyv), T(cu[1].y - t1 * kyv));
-            cu[2] = mk<T>(T(cu[2].x - t0 * kzv), T(cu[2].y - t1 * kzv));
-        } else {
-            cu[0] = cu[1] = cu[2] = mk<T>(T(0), T(0));
-        }
-        // integrating-factor RK stage
-        const double dt = sp.dt;
-        if (STAGE == 1) {
-            if (k2 <= g.kM2) {
-                const double f0 = exp(-sp.nu * k2 * dt);
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const C2<T> w0 = v0[c * PS + off];
-                    dst[c * PS + off] = mk<T>(T((w0.x + dt * cu[c].x) * f0), T((w0.y + dt * cu[c].y) * f0));
-                }
+                for (int c = 0; c < 3; c++) a[c] = mk<T>(T(res[c][i].x * flt), T(res[c][i].y * flt));
             } else {
 #pragma unroll
-                for (int c = 0; c < 3; c++) dst[c * PS + off] = mk<T>(T(0), T(0));
+                for (int c = 0; c < 3; c++) a[c] = k2 >= g.kM2 ? mk<T>(T(0), T(0)) : res[c][i];
             }
-        } else if (STAGE == 2) {
-            if (k2 <= g.kM2) {
-                const double f0 = exp(-sp.nu * k2 * dt / 2);
-                const double f1 = exp(sp.nu * k2 * dt / 2);
+            // curl: i k x a
+            C2<T> cu[3];
+            cu[0] = mk<T>(T(-(kyv * a[2].y - kzv * a[1].y)), T(kyv * a[2].x - kzv * a[1].x));
+            cu[1] = mk<T>(T(-(kzv * a[0].y - kx * a[2].y)), T(kzv * a[0].x - kx * a[2].x));
+            cu[2] = mk<T>(T(-(kx * a[1].y - kyv * a[0].y)), T(kx * a[1].x - kyv * a[0].x));
+            // forcing with the stage's source vorticity
+            // (the wavenumber's root is taken near the band only)
+            if ((sp.forcing == 1 || sp.forcing == 3) && k2 <= fk1sq) {
+                const double kn = sqrt(k2);
+                if (sp.fk0 <= kn && sp.fk1 >= kn) {
+                    const double amp = sp.forcing == 1 ? sp.famp : sp.famp_dev[STAGE - 1];
 #pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const C2<T> w0 = v0[c * PS + off];
-                    const C2<T> w1 = vp[c * PS + off];
-                    dst[c * PS + off] = mk<T>(T((3 * w0.x * f0 + (w1.x + dt * cu[c].x) * f1) * 0.25),
-                                              T((3 * w0.y * f0 + (w1.y + dt * cu[c].y) * f1) * 0.25));
+                    for (int c = 0; c < 3; c++) {
+                        const C2<T> s = STAGE == 1 ? w0[c] : w1[c];
+                        cu[c] = mk<T>(T(cu[c].x + amp * double(s.x) * 1.0), T(cu[c].y + amp * double(s.y) * 1.0));
+                    }
+                }
+            } else if (sp.forcing == 2) {
+                if (kxi == 0 && kz == 0 && (ky == sp.fmode || ky == N - sp.fmode))
+                    cu[2].x = T(cu[2].x - sp.famp * 1.0 / 2);
+            }
+            // force_divfree (zero at k = 0), then the integrating-factor RK stage
+            const double ik2 = k2 > 0 ? 1.0 / k2 : 0.0;  // one division, then products
+            if (k2 > 0) divfree<T>(cu, kx, kyv, kzv, ik2);
+            else cu[0] = cu[1] = cu[2] = mk<T>(T(0), T(0));
+            const double f0 = if_of(ifxz, ify[0][ky]);
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                if constexpr (STAGE == 1) {
+                    nv[c] = mk<T>(T((w0[c].x + dt * cu[c].x) * f0), T((w0[c].y + dt * cu[c].y) * f0));
+                } else if constexpr (STAGE == 2) {
+                    const double f1 = if_of(ifxz1, ify[STAGE - 1][ky]);
+                    nv[c] = mk<T>(T((3 * w0[c].x * f0 + (w1[c].x + dt * cu[c].x) * f1) * 0.25),
+                                  T((3 * w0[c].y * f0 + (w1[c].y + dt * cu[c].y) * f1) * 0.25));
+                } else {
+                    const double f3 = f0 * (1.0 / 3);  // products instead of six divisions by 3
+                    nv[c] = mk<T>(T((w0[c].x * f0 + 2 * (w1[c].x + dt * cu[c].x)) * f3),
+                                  T((w0[c].y * f0 + 2 * (w1[c].y + dt * cu[c].y)) * f3));
                 }
             }
+            if constexpr (STAGE == 3) {
+                // final force_divfree of the new vorticity
+                if (k2 > 0) divfree<T>(nv, kx, kyv, kzv, ik2);
+                else nv[0] = nv[1] = nv[2] = mk<T>(T(0), T(0));
+            }
+        } else if (STAGE == 3 && full) {
+            // v0 there is kept, with the final projection (k2 > 0)
+#pragma unroll
+            for (int c = 0; c < 3; c++) nv[c] = w0[c];
+            divfree<T>(nv, kx, kyv, kzv, 1.0 / k2);
         } else {
-            C2<T> nv[3];
-            if (k2 <= g.kM2) {
-                const double f0 = exp(-sp.nu * k2 * dt * 0.5);
-                const double f3 = f0 * (1.0 / 3);  // products instead of six divisions by 3
-#pragma unroll
-                for (int c = 0; c < 3; c++) {
-                    const C2<T> w0 = v0[c * PS + off];
-                    const C2<T> w2 = vp[c * PS + off];
-                    nv[c] = mk<T>(T((w0.x * f0 + 2 * (w2.x + dt * cu[c].x)) * f3),
-                                  T((w0.y * f0 + 2 * (w2.y + dt * cu[c].y)) * f3));
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < 3; c++) nv[c] = v0[c * PS + off];
-            }
-            // final force_divfree of the new vorticity
-            if (k2 > 0) {
-                const double ik2 = 1.0 / k2;
-                const T t0 = T((kx * nv[0].x + kyv * nv[1].x + kzv * nv[2].x) * ik2);
-                const T t1 = T((kx * nv[0].y + kyv * nv[1].y + kzv * nv[2].y) * ik2);
-                nv[0] = mk<T>(T(nv[0].x - t0 * kx), T(nv[0].y - t1 * kx));
-                nv[1] = mk<T>(T(nv[1].x - t0 * kyv), T(nv[1].y - t1 * kyv));
-                nv[2] = mk<T>(T(nv[2].x - t0 * kzv), T(nv[2].y - t1 * kzv));
-            } else {
-                nv[0] = nv[1] = nv[2] = mk<T>(T(0), T(0));
-            }
-#pragma unroll
-            for (int c = 0; c < 3; c++) dst[c * PS + off] = nv[c];
+            nv[0] = nv[1] = nv[2] = mk<T>(T(0), T(0));
+            write = false;
         }
+        if (write) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) at_off<T>(dst + c * PS, off) = nv[c];
+        }
+        if constexpr (STAGE < 3) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) res[c][i] = nv[c];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (STAGE < 3) {
+        // the first inverse pass of the next stage: register element e of
+        // its input is row F::in_row(e), which element i of the forward
+        // output holds (both are rows grp + G m)
+        using FI = RegFft<T, N, B, B, NT, +1>;
+        using P = typename F::P;
+        constexpr int R0 = P::radix(0), RL = P::radix(P::nstages - 1);
+        C2<T> wr[3][E];
+        sfor<0, E>([&](auto e) {
+            constexpr int m = e / R0 + (e % R0) * (E / R0);
+            constexpr int i = (m % (E / RL)) * RL + m / (E / RL);
+#pragma unroll
+            for (int c = 0; c < 3; c++) wr[c][e] = res[c][i];
+        });
+        bs_inverse_y<T, N, 0, FI, E>(wr, lds, tw, w, grp, b, kxi, kz, g);
     }
 }
 

@@ -1,0 +1,103 @@
+"""The step's band table (pencils outside the dealiasing sphere are neither
+transformed nor moved), its whole-spectrum form for unprojected data, the
+kx = 0 plane factor that stands in for the symmetrized velocity, and both
+forms of the integrating factor, against the CPU oracle.
+
+Tolerance: relative L2 1e-11 after a few FP64 steps, that of the other FP64
+step tests (rounding of 27 transforms a step, about 1e-15 each).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-11
+
+
+def rel(a, b):
+    return np.linalg.norm((a - b).ravel()) / max(np.linalg.norm(b.ravel()), 1e-300)
+
+
+def spectrum(n, seed):
+    """Every mode but the unstored kx = n/2 ones, not conjugate-symmetric on
+    kx = 0: what a caller may put without a projection."""
+    rng = np.random.default_rng(seed)
+    shp = (n, n, n // 2 + 1, 3)
+    a = rng.standard_normal(shp) + 1j * rng.standard_normal(shp)
+    kx = np.arange(n // 2 + 1)
+    k1 = np.where(np.arange(n) <= n // 2, np.arange(n), np.arange(n) - n)
+    k2 = k1[:, None, None] ** 2 + k1[None, :, None] ** 2 + kx[None, None, :] ** 2
+    a *= (1.0 / (1.0 + k2))[..., None]
+    a[:, :, n // 2] = 0
+    return a
+
+
+@pytest.mark.parametrize("n, dealias, projected, dk, nu", [
+    (16, "SMOOTH", False, (1.0, 1.0, 1.0), 0.02),
+    (32, "SMOOTH", True, (1.0, 1.0, 1.0), 0.02),
+    (32, "TWO_THIRDS", False, (1.0, 1.0, 1.0), 0.02),
+    (48, "SMOOTH", False, (1.0, 1.0, 1.0), 0.02),
+    (48, "TWO_THIRDS", True, (1.0, 1.0, 1.0), 0.02),
+    # ky = n/2 and kz = n/2 inside the sphere (kx = n/2, which is not stored, never is)
+    (64, "SMOOTH", True, (1.0, 0.5, 0.75), 0.02),
+    (64, "TWO_THIRDS", True, (1.25, 1.0, 0.5), 0.02),
+    (32, "SMOOTH", True, (1.0, 1.0, 1.0), 2.0),     # damping of the last modes above exp(-1/2) per step
+    (128, "TWO_THIRDS", True, (1.0, 1.0, 1.0), 0.02),
+])
+def test_step(oracle, n, dealias, projected, dk, nu):
+    import bfps_amd as B
+    w0 = spectrum(n, n)
+    print("case: band n=%d %s projected=%s dk=%s nu=%g" % (n, dealias, projected, dk, nu), flush=True)
+    fs = B.vorticity_equation("t", n, dkx=dk[0], dky=dk[1], dkz=dk[2], precision="double", dealias=dealias)
+    fs.nu, fs.famplitude, fs.forcing_type = nu, 0.3, "linear"
+    o = oracle.Solver(n, precision="double", dealias=dealias, dk=dk)
+    o.set_physics(nu, "linear", 0.3, 2.0, 4.0)
+    o.set_cfield("vorticity", w0)
+    if projected:
+        fs.io_checkpoint(read=True, data=w0)
+        o.io_projection()
+    else:
+        fs.cvorticity = w0
+    for _ in range(3):
+        fs.step(0.005)
+        o.step(0.005)
+    e = rel(fs.cvorticity, o.get_cfield("vorticity"))
+    print("  rel", e, flush=True)
+    assert e < TOL
+
+
+def test_put_switches_the_table(oracle):
+    """An unprojected put, then a projection, then steps: each form in turn,
+    and the same in a box of an ensemble beside a projected one."""
+    import bfps_amd as B
+    n, dt = 32, 0.005
+    w = spectrum(n, 5)
+
+    def reference(projected):
+        o = oracle.Solver(n, precision="double")
+        o.set_physics(0.02, "none", 0.0, 2.0, 4.0)
+        o.set_cfield("vorticity", w)
+        if projected:
+            o.io_projection()
+        o.step(dt)
+        return o.get_cfield("vorticity")
+
+    fs = B.vorticity_equation("t", n, precision="double")
+    fs.nu, fs.forcing_type = 0.02, "none"
+    for projected in (True, False, True):
+        if projected:
+            fs.io_checkpoint(read=True, data=w)
+        else:
+            fs.cvorticity = w
+        fs.step(dt)
+        assert rel(fs.cvorticity, reference(projected)) < TOL
+    ens = B.ensemble([n, n], precision="double")
+    for projected in (True, False, True):
+        for i, b in enumerate(ens.boxes):
+            b.nu, b.forcing_type = 0.02, "none"
+            if i == 0 or projected:
+                b.io_checkpoint(read=True, data=w)
+            else:
+                b.cvorticity = w
+        ens.step(dt, with_particles=False)
+        assert rel(ens.boxes[0].cvorticity, reference(True)) < TOL
+        assert rel(ens.boxes[1].cvorticity, reference(projected)) < TOL
