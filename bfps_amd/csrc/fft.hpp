@@ -335,6 +335,9 @@ struct RegFft {
     }
     static BFPSH_DEV int in_row(int g, int e) { return in_row_s(0, g, e); }
     static BFPSH_DEV int out_row(int g, int e) { return out_row_s(S - 1, g, e); }
+    // both are rows g + G m, with m of element e:
+    static constexpr int in_m(int e) { return e / P::radix(0) + (e % P::radix(0)) * (E / P::radix(0)); }
+    static constexpr int out_m(int e) { return e / P::radix(S - 1) + (e % P::radix(S - 1)) * (E / P::radix(S - 1)); }
 
     template <int s>
     static BFPSH_DEV void compute_stage(C2<T> (&v)[E], const C2<T>* __restrict__ tw, int g) {
@@ -356,19 +359,26 @@ struct RegFft {
         }
     }
 
-    // v: stage-0 inputs on entry, last-stage outputs on exit.  The LDS tile
-    // is free again when this returns (trailing barrier included only when
-    // an exchange happened).
-    static BFPSH_DEV void run(C2<T> (&v)[E], C2<T>* lds, const C2<T>* __restrict__ tw, int g, int b) {
+    // v: stage-0 inputs on entry, last-stage outputs on exit.
+    // NBUF = 1: one LDS tile, which an exchange may overwrite only after every
+    // wave has read the one before; `tail`: also after the last exchange, for
+    // a caller that uses the tile again.
+    // NBUF = 2: exchanges alternate between two tiles (cur: the next one), so
+    // that the barrier of one exchange also frees the tile of the one before
+    // and each costs one barrier instead of two.
+    template <int NBUF, bool tail>
+    static BFPSH_DEV void run(C2<T> (&v)[E], C2<T>* lds, const C2<T>* __restrict__ tw, int g, int b, int& cur) {
         sfor<0, S>([&](auto s) {
             compute_stage<s>(v, tw, g);
             if constexpr (s + 1 < S) {
+                C2<T>* buf = NBUF == 2 ? lds + cur * (N * LS) : lds;
 #pragma unroll
-                for (int e = 0; e < E; e++) lds[out_row_s(s, g, e) * LS + b] = v[e];
+                for (int e = 0; e < E; e++) buf[out_row_s(s, g, e) * LS + b] = v[e];
                 __syncthreads();
 #pragma unroll
-                for (int e = 0; e < E; e++) v[e] = lds[in_row_s(s + 1, g, e) * LS + b];
-                __syncthreads();
+                for (int e = 0; e < E; e++) v[e] = buf[in_row_s(s + 1, g, e) * LS + b];
+                if constexpr (NBUF == 2) cur ^= 1;
+                else if constexpr (tail || s + 2 < S) __syncthreads();
             }
         });
     }

@@ -142,8 +142,8 @@ struct Impl {
 
     // The pass autotuner: for each pass kind, the shape held by the wisdom
     // when a search of at least this rigor chose it (any wisdom for
-    // ESTIMATE), else the fastest of all compiled shapes timed on one
-    // scratch plane (ESTIMATE without wisdom: the built-in shape), as FFTW's
+    // ESTIMATE), else the fastest of all compiled shapes timed on the work
+    // planes (ESTIMATE without wisdom: the built-in shape), as FFTW's
     // planner searches its algorithms under the reference's plan rigor
     // (bfps/cpp/fftw_interface.hpp:30-35) and reuses its wisdom.
     static int tune_passes(bfpsh_ctx* ctx, int rigor) {
@@ -152,7 +152,6 @@ struct Impl {
             int r = ensure_work(ctx, 6);
             if (r) return r;
         }
-        void* scratch = nullptr;
         hipEvent_t a = nullptr, b = nullptr;
         int rc = BFPSH_OK;
         for (int kind = 0; kind < BFPSH_PASS_KINDS && rc == BFPSH_OK; kind++) {
@@ -167,11 +166,12 @@ struct Impl {
                 continue;
             }
             if (rigor == BFPSH_ESTIMATE) continue;
-            if (!scratch) {
-                const size_t bytes = ctx->ps * sizeof(CT);
-                if (hipMalloc(&scratch, bytes) != hipSuccess || hipMemsetAsync(scratch, 0, bytes, ctx->stream) != hipSuccess ||
+            if (!a) {
+                // (transforms of whatever the work planes hold would grow
+                // without bound over the trials)
+                if (hipMemsetAsync(ctx->work, 0, 3 * ctx->ps * sizeof(CT), ctx->stream) != hipSuccess ||
                     hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) {
-                    rc = fail(ctx, BFPSH_EHIP, "pass autotuner: scratch plane or events");
+                    rc = fail(ctx, BFPSH_EHIP, "pass autotuner: work planes or events");
                     break;
                 }
             }
@@ -180,8 +180,10 @@ struct Impl {
             int bestv = 0;
             for (int v = 0; v < sh.n && rc == BFPSH_OK; v++) {
                 const CT* tw = (const CT*)ctx->tw;
-                // one launch of shape v: a plain pass over the scratch plane;
-                // the first pass from cvorticity into the work planes; the
+                // one launch of shape v: a plain pass over three work planes
+                // (one plane would stay in the last-level cache, where other
+                // shapes win), the z passes within the band as the step runs
+                // them; the first pass from cvorticity into the work planes; the
                 // last pass of stage 1 from the work planes into v1 (which
                 // every step writes before it reads it) and back into them
                 auto run = [&]() {
@@ -195,8 +197,9 @@ struct Impl {
                         y3_fn(1, v)(ctx->stream, (CT*)ctx->work, (const CT*)ctx->v0, (const CT*)ctx->v1,
                                     (CT*)ctx->v1, tw, band(ctx), ctx->outside, geom(ctx), sp);
                     } else {
-                        pass_fn(kind, v)(ctx->stream, static_cast<CT*>(scratch), pass_estride(kind),
-                                         pass_ostride(kind), tw, 1, 0, 1, nullptr);
+                        const bool z = kind == BFPSH_PASS_Z_INV || kind == BFPSH_PASS_Z_FWD;
+                        pass_fn(kind, v)(ctx->stream, (CT*)ctx->work, pass_estride(kind), pass_ostride(kind), tw, 3, 0,
+                                         1, z ? band(ctx) : nullptr);
                     }
                 };
                 run();  // warm-up
@@ -228,10 +231,6 @@ struct Impl {
         }
         if (a) (void)hipEventDestroy(a);
         if (b) (void)hipEventDestroy(b);
-        if (scratch) {
-            (void)hipStreamSynchronize(ctx->stream);
-            (void)hipFree(scratch);
-        }
         return rc;
     }
 

@@ -131,20 +131,14 @@ struct Cfg {
 template <int N> BFPSH_DEV size_t crow(size_t row) { return (row / N) * row_stride(N) + (row % N) * (N / 2); }
 template <int N> BFPSH_DEV size_t rrow(size_t row) { return (row / N) * 2 * row_stride(N) + (row % N) * N; }
 
-// Element (row n of stride YS, column col) of a plane: byte offset in 32 bits
-// where a plane is smaller than 4 GiB, so that one register of offset serves
-// every plane from its base in scalar registers
-template <typename T, int N> BFPSH_DEV auto yoff(int n, uint32_t col) {
-    constexpr uint64_t bytes = plane_size(N) * sizeof(C2<T>);
-    if constexpr (bytes < (uint64_t(1) << 32))
-        return uint32_t(uint32_t(n) * uint32_t(row_stride(N)) + col) * uint32_t(sizeof(C2<T>));
-    else
-        return (uint64_t(n) * row_stride(N) + col) * sizeof(C2<T>);
-}
-template <typename T, class O> BFPSH_DEV C2<T>& at_off(C2<T>* p, O off) {
+// Element at a byte offset of 32 bits from a pointer that is uniform over the
+// workgroup: the pointer stays in scalar registers and one vector register of
+// offset serves every row g + G m (the G m rows are part of the pointer) and
+// every plane.  A thread's own offset (row g, column) stays below 2^31 bytes.
+template <typename T> BFPSH_DEV C2<T>& at_off(C2<T>* p, uint32_t off) {
     return *reinterpret_cast<C2<T>*>(reinterpret_cast<char*>(p) + off);
 }
-template <typename T, class O> BFPSH_DEV const C2<T>& at_off(const C2<T>* p, O off) {
+template <typename T> BFPSH_DEV const C2<T>& at_off(const C2<T>* p, uint32_t off) {
     return *reinterpret_cast<const C2<T>*>(reinterpret_cast<const char*>(p) + off);
 }
 
@@ -224,13 +218,23 @@ BFPSH_DEV C2<T> biot_savart(int cu, C2<T> a0, C2<T> a1, C2<T> a2, double kx, dou
     return u;
 }
 
+// offset of row g, column kxi of a y pencil
+template <typename T, int N> BFPSH_DEV uint32_t y_off(int g, int kxi) {
+    return (uint32_t(g) * uint32_t(row_stride(N)) + uint32_t(kxi)) * uint32_t(sizeof(C2<T>));
+}
+
+// LDS tiles of the fused y passes: two (one barrier an exchange, nine
+// transforms a workgroup) wherever two tiles take at most the 128 KB that
+// leave the integrating-factor table its room
+template <typename T, int N> constexpr int fused_bufs(int b) { return N * b * int(sizeof(C2<T>)) <= 65536 ? 2 : 1; }
+
 // Fields of the column (kxi, kz) from its vorticity wr (element e at row
 // F::in_row(grp, e)), inverse-transformed along y into o + f PS, f < NF.
-template <typename T, int N, int MODE, class F, int E>
-BFPSH_DEV void bs_inverse_y(C2<T> (&wr)[3][E], C2<T>* lds, const C2<T>* __restrict__ tw, C2<T>* o, int grp, int b,
-                            int kxi, int kz, const Geom& g) {
-    constexpr size_t PS = plane_size(N);
-    const uint32_t col = uint32_t(kz) * uint32_t(N / 2) + uint32_t(kxi);
+template <typename T, int N, int MODE, class F, int E, int NBUF>
+BFPSH_DEV void bs_inverse_y(C2<T> (&wr)[3][E], C2<T>* lds, int cur, const C2<T>* __restrict__ tw, C2<T>* o, int grp,
+                            int b, int kxi, int kz, const Geom& g) {
+    constexpr size_t PS = plane_size(N), GS = F::G * row_stride(N);
+    o += size_t(kz) * (N / 2);
     constexpr int NF = BsOut<MODE>::NF;
     const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
     // Velocity-type fields in a runtime loop (register arrays indexed by
@@ -270,20 +274,20 @@ BFPSH_DEV void bs_inverse_y(C2<T> (&wr)[3][E], C2<T>* lds, const C2<T>* __restri
                 v[e] = u;
             }
         }
-        F::run(v, lds, tw, gq, b);
+        F::template run<NBUF, true>(v, lds, tw, gq, b, cur);
         C2<T>* of = o + size_t(f) * PS;
 #pragma unroll
-        for (int e = 0; e < E; e++) at_off<T>(of, yoff<T, N>(F::out_row(gq, e), col)) = v[e];
+        for (int e = 0; e < E; e++) at_off<T>(of + F::out_m(e) * GS, y_off<T, N>(gq, kxi)) = v[e];
     }
     if constexpr (MODE == 0) {
         sfor<0, 3>([&](auto cc) {
             constexpr int c = cc;
             int gq = grp, t0 = 0;
             asm volatile("" : "+v"(gq), "+s"(t0));
-            F::run(wr[c], lds, tw + t0, gq, b);
+            F::template run<NBUF, c != 2>(wr[c], lds, tw + t0, gq, b, cur);
             C2<T>* of = o + size_t(3 + c) * PS;
 #pragma unroll
-            for (int e = 0; e < E; e++) at_off<T>(of, yoff<T, N>(F::out_row(gq, e), col)) = wr[c][e];
+            for (int e = 0; e < E; e++) at_off<T>(of + F::out_m(e) * GS, y_off<T, N>(gq, kxi)) = wr[c][e];
         });
     }
 }
@@ -299,9 +303,10 @@ k_bs_inv_y(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __
     w += blockIdx.z * bstride;
     out += blockIdx.z * bstride;
     constexpr int B = B_, E = E_, NT = (N / E_) * B_, NXH = CF::NXH;
-    constexpr size_t PS = plane_size(N);
+    constexpr size_t PS = plane_size(N), GS = (NT / B) * row_stride(N);
     using F = RegFft<T, N, B, B, NT, +1>;
-    __shared__ C2<T> lds[N * B];
+    constexpr int NBUF = fused_bufs<T, N>(B);
+    __shared__ C2<T> lds[NBUF * N * B];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
     int tile, kz;
@@ -309,7 +314,7 @@ k_bs_inv_y(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __
     if (min(kz, N - kz) > zl[tile * B]) return;  // uniform: the whole tile lies outside the sphere
     const int kxi = tile * B + b;
     const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
-    const uint32_t col = uint32_t(kz) * uint32_t(NXH) + uint32_t(kxi);
+    w += size_t(kz) * NXH;
     C2<T> wr[3][E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
@@ -317,9 +322,9 @@ k_bs_inv_y(const C2<T>* __restrict__ w, C2<T>* __restrict__ out, const C2<T>* __
         const double kyv = kwave(n, N, g.dky);
         const bool in = full || kx * kx + kyv * kyv + kzv * kzv <= g.kM2;
 #pragma unroll
-        for (int c = 0; c < 3; c++) wr[c][e] = in ? at_off<T>(w + c * PS, yoff<T, N>(n, col)) : mk<T>(T(0), T(0));
+        for (int c = 0; c < 3; c++) wr[c][e] = in ? at_off<T>(w + c * PS + F::in_m(e) * GS, y_off<T, N>(grp, kxi)) : mk<T>(T(0), T(0));
     }
-    bs_inverse_y<T, N, MODE, F, E>(wr, lds, tw, out, grp, b, kxi, kz, g);
+    bs_inverse_y<T, N, MODE, F, E, NBUF>(wr, lds, 0, tw, out, grp, b, kxi, kz, g);
 }
 
 // ------------------------------------------------------------ generic strided pass (in place)
@@ -352,15 +357,19 @@ k_pass(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __
     }
     // blockIdx.z = box * planes + plane (boxes bstride elements apart)
     const int box = blockIdx.z / planes, plane = blockIdx.z % planes;
-    C2<T>* base = data + box * bstride + plane * PS + blockIdx.y * ostride + blockIdx.x * B + b;
+    C2<T>* base = data + box * bstride + plane * PS + blockIdx.y * ostride + blockIdx.x * B;
+    const uint32_t off = (uint32_t(grp) * uint32_t(estride) + uint32_t(b)) * uint32_t(sizeof(C2<T>));
+    const size_t gs = F::G * estride;
     C2<T> v[E];
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int n = F::in_row(grp, e);
-        if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? base[n * estride] : mk<T>(T(0), T(0));
-        else v[e] = base[n * estride];
+        const C2<T>* row = base + F::in_m(e) * gs;
+        if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? at_off<T>(row, off) : mk<T>(T(0), T(0));
+        else v[e] = at_off<T>(row, off);
     }
-    F::run(v, lds, tw, grp, b);
+    int cur = 0;
+    F::template run<1, false>(v, lds, tw, grp, b, cur);
     if constexpr (BAND && SIGN < 0) {
         // (not to be sunk into the conditional stores)
 #pragma unroll
@@ -369,7 +378,7 @@ k_pass(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>* __
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const int n = F::out_row(grp, e);
-        if (!(BAND && SIGN < 0) || in_band<N>(n, lim)) base[n * estride] = v[e];
+        if (!(BAND && SIGN < 0) || in_band<N>(n, lim)) at_off<T>(base + F::out_m(e) * gs, off) = v[e];
     }
 }
 
@@ -395,14 +404,17 @@ k_pass_pp(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>*
         const int x = t % ntx, r = t / ntx, y = r % nty, zp = r / nty;
         const int box = zp / planes, plane = zp % planes;
         lim = BAND ? zl[x * B + b] : N;
-        return data + box * bstride + plane * PS + size_t(y) * ostride + size_t(x) * B + b;
+        return data + box * bstride + plane * PS + size_t(y) * ostride + size_t(x) * B;
     };
+    const uint32_t off = (uint32_t(grp) * uint32_t(estride) + uint32_t(b)) * uint32_t(sizeof(C2<T>));
+    const size_t gs = F::G * estride;
     auto load = [&](const C2<T>* p, int lim, C2<T> (&v)[E]) {
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int n = F::in_row(grp, e);
-            if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? p[n * estride] : mk<T>(T(0), T(0));
-            else v[e] = p[n * estride];
+            const C2<T>* row = p + F::in_m(e) * gs;
+            if constexpr (BAND && SIGN > 0) v[e] = in_band<N>(n, lim) ? at_off<T>(row, off) : mk<T>(T(0), T(0));
+            else v[e] = at_off<T>(row, off);
         }
     };
     int t = blockIdx.x;
@@ -419,11 +431,12 @@ k_pass_pp(C2<T>* __restrict__ data, size_t estride, size_t ostride, const C2<T>*
             pn = base_of(tn, nlim);
             load(pn, nlim, nxt);
         }
-        F::run(cur, lds, tw, grp, b);
+        int buf = 0;
+        F::template run<1, true>(cur, lds, tw, grp, b, buf);
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const int n = F::out_row(grp, e);
-            if (!BAND || (SIGN > 0 ? lim >= 0 : in_band<N>(n, lim))) p[n * estride] = cur[e];
+            if (!BAND || (SIGN > 0 ? lim >= 0 : in_band<N>(n, lim))) at_off<T>(p + F::out_m(e) * gs, off) = cur[e];
         }
         if (!more) break;
 #pragma unroll
@@ -934,9 +947,10 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     }
     const StepParams sp = BATCH ? spb[blockIdx.z] : sp0;
     constexpr int B = B_, E = E_, NT = (N / E_) * B_, NXH = CF::NXH;
-    constexpr size_t PS = plane_size(N);
+    constexpr size_t PS = plane_size(N), GS = (NT / B) * row_stride(N);
     using F = RegFft<T, N, B, B, NT, -1>;
-    __shared__ C2<T> lds[N * B];
+    constexpr int NBUF = fused_bufs<T, N>(B);
+    __shared__ C2<T> lds[NBUF * N * B];
     __shared__ double ify[STAGE == 2 ? 2 : 1][N];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
@@ -948,13 +962,16 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     if (kza > zl[tile * B]) return;  // uniform: the whole tile lies outside the sphere
     const int kxi = tile * B + b;
     const bool col_in = kza <= zl[kxi];
-    const uint32_t col = uint32_t(kz) * uint32_t(NXH) + uint32_t(kxi);
+    const size_t kzs = size_t(kz) * NXH;
+    v0 += kzs;
+    vp += kzs;
+    dst += kzs;
     C2<T> res[3][E];
 #pragma unroll
     for (int c = 0; c < 3; c++)
 #pragma unroll
         for (int e = 0; e < E; e++)
-            res[c][e] = col_in ? at_off<T>(w + c * PS, yoff<T, N>(F::in_row(grp, e), col)) : mk<T>(T(0), T(0));
+            res[c][e] = col_in ? at_off<T>(w + c * PS + kzs + F::in_m(e) * GS, y_off<T, N>(grp, kxi)) : mk<T>(T(0), T(0));
     const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
     const double dt = sp.dt, nud = sp.nu * dt * (STAGE == 1 ? 1.0 : 0.5);
     const bool slow = fabs(nud) * g.kM2 < 0.5;  // uniform
@@ -972,11 +989,12 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     // per component, so that twiddles and LDS addresses are not held across,
     // and opaque results, so that the last butterflies are not sunk into the
     // conditional code below (which would keep all their inputs alive)
+    int cur = 0;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         int gq = grp, t0 = 0;
         asm volatile("" : "+v"(gq), "+s"(t0));
-        F::run(res[c], lds, tw + t0, gq, b);
+        F::template run<NBUF, true>(res[c], lds, tw + t0, gq, b, cur);
 #pragma unroll
         for (int e = 0; e < E; e++) asm volatile("" : "+v"(res[c][e].x), "+v"(res[c][e].y));
     }
@@ -992,11 +1010,12 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
         const int ky = F::out_row(gq, i);
         const double kyv = kwave(ky, N, g.dky);
         if (kx * kx + kyv * kyv + kzv * kzv <= g.kM2 || (STAGE == 3 && full)) {
-            const auto off = yoff<T, N>(ky, col);
+            const uint32_t off = y_off<T, N>(gq, kxi);
+            const size_t row = F::out_m(i) * GS;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
-                q0[c] = at_off<T>(v0 + c * PS, off);
-                if (STAGE > 1) q1[c] = at_off<T>(vp + c * PS, off);
+                q0[c] = at_off<T>(v0 + c * PS + row, off);
+                if (STAGE > 1) q1[c] = at_off<T>(vp + c * PS + row, off);
             }
         }
     };
@@ -1011,7 +1030,7 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
         const int ky = F::out_row(gq, i);
         const double kyv = kwave(ky, N, g.dky);
         const double k2 = kx * kx + kyv * kyv + kzv * kzv;
-        const auto off = yoff<T, N>(ky, col);
+        const uint32_t off = y_off<T, N>(gq, kxi);
         C2<T> nv[3];
         bool write = true;
         if (k2 <= g.kM2) {
@@ -1083,7 +1102,7 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
         }
         if (write) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) at_off<T>(dst + c * PS, off) = nv[c];
+            for (int c = 0; c < 3; c++) at_off<T>(dst + c * PS + F::out_m(i) * GS, off) = nv[c];
         }
         if constexpr (STAGE < 3) {
 #pragma unroll
@@ -1096,16 +1115,16 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
         // its input is row F::in_row(e), which element i of the forward
         // output holds (both are rows grp + G m)
         using FI = RegFft<T, N, B, B, NT, +1>;
-        using P = typename F::P;
-        constexpr int R0 = P::radix(0), RL = P::radix(P::nstages - 1);
         C2<T> wr[3][E];
         sfor<0, E>([&](auto e) {
-            constexpr int m = e / R0 + (e % R0) * (E / R0);
-            constexpr int i = (m % (E / RL)) * RL + m / (E / RL);
+            sfor<0, E>([&](auto i) {
+                if constexpr (F::out_m(i) == FI::in_m(e)) {
 #pragma unroll
-            for (int c = 0; c < 3; c++) wr[c][e] = res[c][i];
+                    for (int c = 0; c < 3; c++) wr[c][e] = res[c][i];
+                }
+            });
         });
-        bs_inverse_y<T, N, 0, FI, E>(wr, lds, tw, w, grp, b, kxi, kz, g);
+        bs_inverse_y<T, N, 0, FI, E, NBUF>(wr, lds, cur, tw, w, grp, b, kxi, kz, g);
     }
 }
 

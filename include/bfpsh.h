@@ -70,7 +70,7 @@ int bfpsh_create(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky
  * ESTIMATE takes the shape the pass wisdom holds, else the built-in one;
  * MEASURE and PATIENT take the wisdom's shape when a search of at least
  * their rigor chose it, else time every compiled shape (3 launches each on
- * one scratch plane for MEASURE, 10 for PATIENT) and keep the fastest in
+ * the work planes for MEASURE, 10 for PATIENT) and keep the fastest in
  * the wisdom.  Boxes below 256^3 have one shape.  At MEASURE and PATIENT
  * the first tracer loop or sample of a tracer set also times the velocity
  * loop of each applicable tracer kernel form (column walk, bricks, global
@@ -81,9 +81,9 @@ int bfpsh_create(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky
  * trials). */
 enum { BFPSH_ESTIMATE = 0, BFPSH_MEASURE = 1, BFPSH_PATIENT = 2 };
 /* strided pass kinds: inverse and forward transforms along kz (z) and ky
- * (y), the vorticity step's fused first pass (Biot-Savart + inverse z) and
+ * (y), the vorticity step's fused first pass (Biot-Savart + inverse y) and
  * its fused last pass (forward y + dealias, curl, forcing, projection and
- * the Runge-Kutta update) */
+ * the Runge-Kutta update, with the first pass of the next stage) */
 enum { BFPSH_PASS_Z_INV = 0, BFPSH_PASS_Y_INV = 1, BFPSH_PASS_Z_FWD = 2, BFPSH_PASS_Y_FWD = 3,
        BFPSH_PASS_BS = 4, BFPSH_PASS_Y3 = 5, BFPSH_PASS_KINDS = 6 };
 
@@ -275,10 +275,10 @@ int bfpsh_device_bytes(bfpsh_ctx* ctx, size_t* bytes);
 /* Replaces the plan creation with `plan_rigor` in the field constructor
  * (bfps/cpp/field.cpp:105-118): chooses the tile shape of each strided pass
  * kind of this context by `rigor` (BFPSH_ESTIMATE / MEASURE / PATIENT, see
- * above).  Measuring allocates one scratch plane for the time it runs and,
- * as FFTW_MEASURE overwrites the arrays it plans for, overwrites the
- * context's work planes (the spectral velocity of compute_velocity); the
- * vorticity and the Runge-Kutta stages are left untouched. */
+ * above).  As FFTW_MEASURE overwrites the arrays it plans for, measuring
+ * overwrites the context's work planes (the spectral velocity of
+ * compute_velocity) and the first Runge-Kutta stage, which every step writes
+ * before it reads it; the vorticity is left untouched. */
 int bfpsh_set_plan_rigor(bfpsh_ctx* ctx, int rigor);
 /* The tile shape in use for pass `kind` (BFPSH_PASS_*): e complex values per
  * thread, b columns per tile, persistent = 1 for the form whose workgroups
