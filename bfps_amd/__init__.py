@@ -172,7 +172,7 @@ class vorticity_equation:
 
     # ---------------------------------------------------------------- fields
     def get_cfield(self, which=capi.CVORTICITY):
-        out = np.zeros(self.cshape(), dtype=self.cdtype)
+        out = np.empty(self.cshape(), dtype=self.cdtype)
         capi.check(self._h, capi.load().bfpsh_get_cfield(self._h, which, out.ctypes.data), "get_cfield")
         return out
 
@@ -267,7 +267,7 @@ class vorticity_equation:
 
     def get_rfield(self, which=capi.RVELOCITY):
         nc = 3 if which == capi.RVELOCITY else 9
-        out = np.zeros((self.nz, self.ny, self.nx, nc), dtype=self.rdtype)
+        out = np.empty((self.nz, self.ny, self.nx, nc), dtype=self.rdtype)
         capi.check(self._h, capi.load().bfpsh_get_rfield(self._h, which, out.ctypes.data), "get_rfield")
         return out
 
@@ -383,9 +383,9 @@ class field:
 
     def get(self):
         if self.real_space_representation:
-            out = np.zeros(self.rshape(), dtype=self.fs.rdtype)
+            out = np.empty(self.rshape(), dtype=self.fs.rdtype)
         else:
-            out = np.zeros(self.cshape(), dtype=self.fs.cdtype)
+            out = np.empty(self.cshape(), dtype=self.fs.cdtype)
         capi.check(self.fs.handle, capi.load().bfpsh_field_get(self.fs.handle, self.id,
                                                                int(self.real_space_representation),
                                                                out.ctypes.data), "field_get")
@@ -494,28 +494,31 @@ class particles_system:
                                              None if i is None else i.ctypes.data_as(capi._LP))
         capi.check(self.fs.handle, rc, "particles_put")
 
-    def get(self):
-        pos = np.zeros((self.np, 3))
-        rhs = np.zeros((self.nsteps, self.np, 3))
-        idx = np.zeros(self.np, dtype=np.int64)
+    def _get(self, pos=False, rhs=False, idx=False):
+        p = np.empty((self.np, 3)) if pos else None
+        r = np.empty((self.nsteps, self.np, 3)) if rhs else None
+        i = np.empty(self.np, dtype=np.int64) if idx else None
         si = ctypes.c_int()
-        rc = capi.load().bfpsh_particles_get(self.fs.handle, pos.ctypes.data_as(capi._DP),
-                                             rhs.ctypes.data_as(capi._DP), idx.ctypes.data_as(capi._LP),
-                                             ctypes.byref(si))
+        rc = capi.load().bfpsh_particles_get(self.fs.handle, None if p is None else p.ctypes.data_as(capi._DP),
+                                             None if r is None else r.ctypes.data_as(capi._DP),
+                                             None if i is None else i.ctypes.data_as(capi._LP), ctypes.byref(si))
         capi.check(self.fs.handle, rc, "particles_get")
-        return pos, rhs, idx, si.value
+        return p, r, i, si.value
+
+    def get(self):
+        return self._get(True, True, True)
 
     def getParticlesPositions(self):
-        return self.get()[0]
+        return self._get(pos=True)[0]
 
     def getParticlesRhs(self):
-        return self.get()[1]
+        return self._get(rhs=True)[1]
 
     def getParticlesIndexes(self):
-        return self.get()[2]
+        return self._get(idx=True)[2]
 
     def get_step_idx(self):
-        return self.get()[3]
+        return self._get()[3]
 
     def completeLoop(self, dt):
         capi.check(self.fs.handle, capi.load().bfpsh_particles_complete_loop(self.fs.handle, float(dt)),
@@ -524,7 +527,7 @@ class particles_system:
     def sample(self, which="velocity"):
         sel = capi.RVELOCITY if which == "velocity" else capi.RGRADIENT
         nc = 3 if which == "velocity" else 9
-        out = np.zeros((self.np, nc))
+        out = np.empty((self.np, nc))
         rc = capi.load().bfpsh_particles_sample(self.fs.handle, sel, out.ctypes.data_as(capi._DP))
         capi.check(self.fs.handle, rc, "particles_sample")
         return out

@@ -75,7 +75,8 @@ def build(jobs=None, sizes=SIZES, verbose=True, out=None, defines=(), incrementa
     os.makedirs(bdir, exist_ok=True)
     extra = ["-D" + d for d in defines]
     tasks = [(os.path.join(CSRC, "bfpsh.hip"), os.path.join(bdir, "bfpsh.o"), extra),
-             (os.path.join(CSRC, "particles.hip"), os.path.join(bdir, "particles.o"), extra)]
+             (os.path.join(CSRC, "particles.hip"), os.path.join(bdir, "particles.o"), extra),
+             (os.path.join(CSRC, "transfer.hip"), os.path.join(bdir, "transfer.o"), extra)]
     for tn, t in (("f32", "float"), ("f64", "double")):
         for n in sizes:
             tasks.append((os.path.join(CSRC, "impl_inst.hip"),

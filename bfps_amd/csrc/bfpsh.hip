@@ -38,56 +38,6 @@ void build_twiddles(std::vector<unsigned char>& out, int n) {
 
 }  // namespace
 
-// host [ky][kz][kx=N/2+1][nc]{re,im} <-> device planar [c][ky][kz][kx<N/2]
-// (ky rows row_stride(n) complex apart, planes plane_size(n) apart)
-template <typename T>
-static void host_to_planar(const T* h, T* p, int n, int nc = 3) {
-    const int nxh = n / 2 + 1, nxs = n / 2;
-    const size_t ps = plane_size(n);
-    for (size_t yz = 0; yz < size_t(n) * n; yz++)
-        for (int x = 0; x < nxs; x++)
-            for (int c = 0; c < nc; c++) {
-                const size_t d = c * ps + sphys(n, yz * nxs + x);
-                p[d * 2 + 0] = h[((yz * nxh + x) * nc + c) * 2 + 0];
-                p[d * 2 + 1] = h[((yz * nxh + x) * nc + c) * 2 + 1];
-            }
-}
-template <typename T>
-static void planar_to_host(const T* p, T* h, int n, int nc = 3) {
-    const int nxh = n / 2 + 1, nxs = n / 2;
-    const size_t ps = plane_size(n);
-    for (size_t yz = 0; yz < size_t(n) * n; yz++)
-        for (int x = 0; x < nxh; x++)
-            for (int c = 0; c < nc; c++) {
-                T re = 0, im = 0;
-                if (x < nxs) {
-                    const size_t d = c * ps + sphys(n, yz * nxs + x);
-                    re = p[d * 2 + 0];
-                    im = p[d * 2 + 1];
-                }
-                h[((yz * nxh + x) * nc + c) * 2 + 0] = re;
-                h[((yz * nxh + x) * nc + c) * 2 + 1] = im;
-            }
-}
-// host real [z][y][x][nc] <-> device planar [c][y][z][x] (real rows y
-// 2 row_stride(n) reals apart, planes 2 plane_size(n) apart)
-template <typename T>
-static void host_real_to_planar(const T* h, T* p, int n, int nc) {
-    const size_t ps = 2 * plane_size(n), ys = 2 * row_stride(n);
-    for (size_t y = 0; y < size_t(n); y++)
-        for (size_t z = 0; z < size_t(n); z++)
-            for (size_t x = 0; x < size_t(n); x++)
-                for (int c = 0; c < nc; c++) p[c * ps + y * ys + z * n + x] = h[((z * n + y) * n + x) * nc + c];
-}
-template <typename T>
-static void planar_to_host_real(const T* p, T* h, int n, int nc) {
-    const size_t ps = 2 * plane_size(n), ys = 2 * row_stride(n);
-    for (size_t y = 0; y < size_t(n); y++)
-        for (size_t z = 0; z < size_t(n); z++)
-            for (size_t x = 0; x < size_t(n); x++)
-                for (int c = 0; c < nc; c++) h[((z * n + y) * n + x) * nc + c] = p[c * ps + y * ys + z * n + x];
-}
-
 #define CTX_CHECK()                                  \
     do {                                             \
         if (!ctx) return BFPSH_EINVAL;               \
@@ -161,6 +111,8 @@ int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, 
     ctx->dkz = dkz;
     ctx->es = precision == BFPSH_FP32 ? 4 : 8;
     HIPCHK(hipSetDevice(device));
+    bfpsh_transfer_open();
+    ctx->pool_user = true;
     {
         int r = scratch_resolve(ctx, device);
         if (r) return r;
@@ -228,9 +180,6 @@ int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, 
     }
     std::vector<unsigned char> tw;
     if (precision == BFPSH_FP32) build_twiddles<float>(tw, n); else build_twiddles<double>(tw, n);
-    HIPCHK(hipMalloc(&ctx->tw, tw.size()));
-    HIPCHK(hipMemcpyAsync(ctx->tw, tw.data(), tw.size(), hipMemcpyHostToDevice, ctx->stream));
-    ctx->bytes += tw.size();
     // band tables (kernels.hpp): a margin of rounding keeps every mode that
     // the kernels' own test k^2 <= kM^2 could take
     const int nh = n / 2;
@@ -242,9 +191,14 @@ int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, 
         if (zl[x] >= 0) zl[nh] = x;
     }
     ctx->xl = zl[nh];
-    HIPCHK(hipMalloc((void**)&ctx->zl, zl.size() * sizeof(int)));
-    HIPCHK(hipMemcpyAsync(ctx->zl, zl.data(), zl.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-    ctx->bytes += zl.size() * sizeof(int);
+    // twiddles and tables in one buffer
+    const size_t twb = tw.size();
+    tw.resize(twb + zl.size() * sizeof(int));
+    std::memcpy(tw.data() + twb, zl.data(), zl.size() * sizeof(int));
+    HIPCHK(hipMalloc(&ctx->tw, tw.size()));
+    ctx->zl = reinterpret_cast<const int*>(static_cast<char*>(ctx->tw) + twb);
+    HIPCHK(hipMemcpyAsync(ctx->tw, tw.data(), tw.size(), hipMemcpyHostToDevice, ctx->stream));
+    ctx->bytes += tw.size();
     int r = ensure_work(ctx, 6);
     if (r) return r;
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -258,9 +212,9 @@ int bfpsh_destroy(bfpsh_ctx* ctx) {
     if (ctx->stream) {
         (void)hipSetDevice(ctx->device);
         (void)hipStreamSynchronize(ctx->stream);
-        for (void* p : {ctx->v0, ctx->v1, ctx->v2, ctx->work, ctx->ru, ctx->rgrad, ctx->tw, (void*)ctx->zl,
+        for (void* p : {ctx->v0, ctx->v1, ctx->v2, ctx->work, ctx->ru, ctx->rgrad, ctx->tw,
                         (void*)ctx->d_pos, (void*)ctx->d_rhs, (void*)ctx->d_tab, (void*)ctx->d_famp,
-                        (void*)ctx->d_rank, (void*)ctx->d_samp})
+                        (void*)ctx->d_order, (void*)ctx->d_samp})
             if (p && !in_slab(ctx, p)) (void)hipFree(p);
         for (void* p : ctx->fields)
             if (p) (void)hipFree(p);
@@ -269,6 +223,7 @@ int bfpsh_destroy(bfpsh_ctx* ctx) {
         for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
         if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
     }
+    if (ctx->pool_user) bfpsh_transfer_close();
     delete ctx;
     return BFPSH_OK;
 }
@@ -315,12 +270,10 @@ int bfpsh_put_cfield(bfpsh_ctx* ctx, int which, const void* host) {
         if (r) return r;
         dst = ctx->work;
     }
-    const size_t bytes = 3 * ctx->ps * 2 * ctx->es;
-    std::vector<unsigned char> tmp(bytes);
-    if (ctx->prec == BFPSH_FP32) host_to_planar<float>((const float*)host, (float*)tmp.data(), ctx->n);
-    else host_to_planar<double>((const double*)host, (double*)tmp.data(), ctx->n);
-    HIPCHK(hipMemcpyAsync(dst, tmp.data(), bytes, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    {
+        int r = bfpsh_field_from_host(ctx, false, 3, dst, host);
+        if (r) return r;
+    }
     if (which == BFPSH_CVORTICITY) {
         ctx->ru_valid = false;
         ctx->outside = 1;
@@ -361,13 +314,7 @@ int bfpsh_get_cfield(bfpsh_ctx* ctx, int which, void* host) {
     } else {
         return fail(ctx, BFPSH_EINVAL, "bad field selector");
     }
-    const size_t bytes = 3 * ctx->ps * 2 * ctx->es;
-    std::vector<unsigned char> tmp(bytes);
-    HIPCHK(hipMemcpyAsync(tmp.data(), src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (ctx->prec == BFPSH_FP32) planar_to_host<float>((const float*)tmp.data(), (float*)host, ctx->n);
-    else planar_to_host<double>((const double*)tmp.data(), (double*)host, ctx->n);
-    return BFPSH_OK;
+    return bfpsh_field_to_host(ctx, false, 3, src, host);
 }
 
 int bfpsh_get_rfield(bfpsh_ctx* ctx, int which, void* host) {
@@ -376,21 +323,7 @@ int bfpsh_get_rfield(bfpsh_ctx* ctx, int which, void* host) {
     const void* src = which == BFPSH_RVELOCITY ? ctx->ru : (which == BFPSH_RGRADIENT ? ctx->rgrad : nullptr);
     const int nc = which == BFPSH_RVELOCITY ? 3 : 9;
     if (!src) return fail(ctx, BFPSH_ESTATE, "real field not computed");
-    const size_t n = ctx->n, rps = 2 * ctx->ps, rys = 2 * row_stride(ctx->n);
-    std::vector<unsigned char> tmp(nc * rps * ctx->es);
-    HIPCHK(hipMemcpyAsync(tmp.data(), src, tmp.size(), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    // device [c][y][z][x] -> host [z][y][x][c]
-    for (size_t y = 0; y < n; y++)
-        for (size_t z = 0; z < n; z++)
-            for (size_t x = 0; x < n; x++)
-                for (int c = 0; c < nc; c++) {
-                    const size_t di = c * rps + y * rys + z * n + x;
-                    const size_t hi = ((z * n + y) * n + x) * nc + c;
-                    if (ctx->prec == BFPSH_FP32) ((float*)host)[hi] = ((const float*)tmp.data())[di];
-                    else ((double*)host)[hi] = ((const double*)tmp.data())[di];
-                }
-    return BFPSH_OK;
+    return bfpsh_field_to_host(ctx, true, nc, src, host);
 }
 
 int bfpsh_load_projection(bfpsh_ctx* ctx) {
@@ -507,18 +440,8 @@ int bfpsh_field_compute_gradient(bfpsh_ctx* ctx, int src_id, int dst_id) {
 int bfpsh_field_put(bfpsh_ctx* ctx, int id, int real_space, const void* host) {
     CTX_CHECK();
     if (!field_ok(ctx, id) || !host) return fail(ctx, BFPSH_EINVAL, "bad field id or buffer");
-    const int nc = ctx->field_nc[id];
-    const size_t bytes = size_t(nc) * ctx->ps * 2 * ctx->es;
-    std::vector<unsigned char> tmp(bytes, 0);
-    if (real_space) {
-        if (ctx->prec == BFPSH_FP32) host_real_to_planar<float>((const float*)host, (float*)tmp.data(), ctx->n, nc);
-        else host_real_to_planar<double>((const double*)host, (double*)tmp.data(), ctx->n, nc);
-    } else {
-        if (ctx->prec == BFPSH_FP32) host_to_planar<float>((const float*)host, (float*)tmp.data(), ctx->n, nc);
-        else host_to_planar<double>((const double*)host, (double*)tmp.data(), ctx->n, nc);
-    }
-    HIPCHK(hipMemcpyAsync(ctx->fields[id], tmp.data(), bytes, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    int r = bfpsh_field_from_host(ctx, real_space != 0, ctx->field_nc[id], ctx->fields[id], host);
+    if (r) return r;
     ctx->field_real[id] = real_space ? 1 : 0;
     return BFPSH_OK;
 }
@@ -526,19 +449,7 @@ int bfpsh_field_put(bfpsh_ctx* ctx, int id, int real_space, const void* host) {
 int bfpsh_field_get(bfpsh_ctx* ctx, int id, int real_space, void* host) {
     CTX_CHECK();
     if (!field_ok(ctx, id) || !host) return fail(ctx, BFPSH_EINVAL, "bad field id or buffer");
-    const int nc = ctx->field_nc[id];
-    const size_t bytes = size_t(nc) * ctx->ps * 2 * ctx->es;
-    std::vector<unsigned char> tmp(bytes);
-    HIPCHK(hipMemcpyAsync(tmp.data(), ctx->fields[id], bytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (real_space) {
-        if (ctx->prec == BFPSH_FP32) planar_to_host_real<float>((const float*)tmp.data(), (float*)host, ctx->n, nc);
-        else planar_to_host_real<double>((const double*)tmp.data(), (double*)host, ctx->n, nc);
-    } else {
-        if (ctx->prec == BFPSH_FP32) planar_to_host<float>((const float*)tmp.data(), (float*)host, ctx->n, nc);
-        else planar_to_host<double>((const double*)tmp.data(), (double*)host, ctx->n, nc);
-    }
-    return BFPSH_OK;
+    return bfpsh_field_to_host(ctx, real_space != 0, ctx->field_nc[id], ctx->fields[id], host);
 }
 
 int bfpsh_field_copy_from(bfpsh_ctx* ctx, int id, int which) {
@@ -629,22 +540,22 @@ int bfpsh_compute_lagrangian_acceleration(bfpsh_ctx* ctx, int id) {
     return PREC_CALL(lagrangian_acceleration, ctx, ctx->fields[id]);
 }
 
-// Slots in global-index order, on the host (order) and as a rank per slot
-// on the device.  The storage order of tracers never changes (sorting for
-// locality only permutes an index array), so this is set once per put.
+// Slots in global-index order, on the host and on the device.  The storage
+// order of tracers never changes (sorting for locality only permutes an index
+// array), so this is set once per put.
 static int set_order(bfpsh_ctx* ctx) {
     ctx->order.resize(ctx->np);
     std::iota(ctx->order.begin(), ctx->order.end(), int64_t(0));
-    std::stable_sort(ctx->order.begin(), ctx->order.end(),
-                     [&](int64_t a, int64_t b) { return ctx->idx[a] < ctx->idx[b]; });
+    if (!std::is_sorted(ctx->idx.begin(), ctx->idx.end()))
+        std::stable_sort(ctx->order.begin(), ctx->order.end(),
+                         [&](int64_t a, int64_t b) { return ctx->idx[a] < ctx->idx[b]; });
     if (ctx->np == 0) return BFPSH_OK;
-    std::vector<uint32_t> rank(ctx->np);
-    for (int64_t i = 0; i < ctx->np; i++) rank[ctx->order[i]] = uint32_t(i);
-    if (!ctx->d_rank) {
-        HIPCHK(hipMalloc((void**)&ctx->d_rank, ctx->np * sizeof(uint32_t)));
+    std::vector<uint32_t> order(ctx->order.begin(), ctx->order.end());
+    if (!ctx->d_order) {
+        HIPCHK(hipMalloc((void**)&ctx->d_order, ctx->np * sizeof(uint32_t)));
         ctx->bytes += ctx->np * sizeof(uint32_t);
     }
-    HIPCHK(hipMemcpyAsync(ctx->d_rank, rank.data(), ctx->np * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->d_order, order.data(), ctx->np * sizeof(uint32_t), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return BFPSH_OK;
 }
@@ -655,9 +566,9 @@ int bfpsh_particles_create(bfpsh_ctx* ctx, int64_t np, int n, int m, int nsteps,
         return fail(ctx, BFPSH_EINVAL, "bad tracer parameters (n in [1,10], m in [0,2], nsteps in [1,6])");
     if (2 * n + 2 > ctx->n) return fail(ctx, BFPSH_EINVAL, "interpolation stencil wider than the grid");
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    for (void* p : {(void*)ctx->d_pos, (void*)ctx->d_rhs, (void*)ctx->d_tab, (void*)ctx->d_rank, (void*)ctx->d_samp})
+    for (void* p : {(void*)ctx->d_pos, (void*)ctx->d_rhs, (void*)ctx->d_tab, (void*)ctx->d_order, (void*)ctx->d_samp})
         if (p) HIPCHK(hipFree(p));
-    ctx->d_rank = nullptr;
+    ctx->d_order = nullptr;
     ctx->d_samp = nullptr;
     {
         int r = bfpsh_part_release(ctx);
@@ -730,12 +641,9 @@ int bfpsh_particles_get(bfpsh_ctx* ctx, double* pos, double* rhs, int64_t* idx, 
     const int64_t np = ctx->np;
     const std::vector<int64_t>& order = ctx->order;
     if (int64_t(order.size()) != np) return fail(ctx, BFPSH_ESTATE, "tracer state not set (particles_put)");
-    std::vector<double> tmp(np * 3);
     if (pos) {
-        HIPCHK(hipMemcpyAsync(tmp.data(), ctx->d_pos, np * 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
-        for (int64_t i = 0; i < np; i++)
-            for (int d = 0; d < 3; d++) pos[i * 3 + d] = tmp[order[i] * 3 + d];
+        int r = bfpsh_rows_to_host(ctx, ctx->d_pos, 3, pos);
+        if (r) return r;
     }
     if (rhs) {
         for (int h = 0; h < ctx->nsteps; h++) {
@@ -744,11 +652,8 @@ int bfpsh_particles_get(bfpsh_ctx* ctx, double* pos, double* rhs, int64_t* idx, 
                 std::fill(rhs, rhs + np * 3, 0.0);
                 continue;
             }
-            HIPCHK(hipMemcpyAsync(tmp.data(), ctx->d_rhs + size_t(slot) * np * 3, np * 3 * sizeof(double),
-                                  hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(hipStreamSynchronize(ctx->stream));
-            for (int64_t i = 0; i < np; i++)
-                for (int d = 0; d < 3; d++) rhs[(size_t(h) * np + i) * 3 + d] = tmp[order[i] * 3 + d];
+            int r = bfpsh_rows_to_host(ctx, ctx->d_rhs + size_t(slot) * np * 3, 3, rhs + size_t(h) * np * 3);
+            if (r) return r;
         }
     }
     if (idx)
@@ -766,35 +671,19 @@ int bfpsh_particles_complete_loop(bfpsh_ctx* ctx, double dt) {
     return bfpsh_part_loop(ctx, dt);
 }
 
-// out[rank[p]][c] = in[p][c]: device rows into global-index order
-static __global__ void k_rank_rows(const double* __restrict__ in, double* __restrict__ out,
-                                   const uint32_t* __restrict__ rank, int64_t np, int nc) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= np * nc) return;
-    const int64_t p = i / nc;
-    out[int64_t(rank[p]) * nc + (i - p * nc)] = in[i];
-}
-
 // sample `nc` real planes [c][y][z][x] at every tracer; out [np][nc] in
 // global-index order
 static int sample_to_host(bfpsh_ctx* ctx, const void* f, int nc, double* out) {
     if (ctx->np == 0) return BFPSH_OK;
     if (int64_t(ctx->order.size()) != ctx->np) return fail(ctx, BFPSH_ESTATE, "tracer state not set (particles_put)");
     if (!ctx->d_samp) {
-        const size_t bytes = size_t(ctx->np) * 9 * 2 * sizeof(double);
+        const size_t bytes = size_t(ctx->np) * 9 * sizeof(double);
         HIPCHK(hipMalloc((void**)&ctx->d_samp, bytes));
         ctx->bytes += bytes;
     }
-    double* raw = ctx->d_samp;
-    double* ranked = ctx->d_samp + size_t(ctx->np) * 9;
-    int r = bfpsh_part_sample(ctx, f, nc, raw);
+    int r = bfpsh_part_sample(ctx, f, nc, ctx->d_samp);
     if (r) return r;
-    const int64_t tot = ctx->np * nc;
-    LAUNCH("rank_rows", (k_rank_rows<<<unsigned((tot + 255) / 256), 256, 0, ctx->stream>>>(raw, ranked, ctx->d_rank,
-                                                                                          ctx->np, nc)));
-    HIPCHK(hipMemcpyAsync(out, ranked, size_t(tot) * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return BFPSH_OK;
+    return bfpsh_rows_to_host(ctx, ctx->d_samp, nc, out);
 }
 
 int bfpsh_particles_sample(bfpsh_ctx* ctx, int which, double* out) {

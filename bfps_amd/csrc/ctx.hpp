@@ -44,7 +44,8 @@ struct bfpsh_ctx {
     void* ru = nullptr;            // real velocity, 3 planes [y][z][x]
     void* rgrad = nullptr;         // real gradient, 9 planes
     void* tw = nullptr;            // twiddles exp(-2 pi i t / N), N complex
-    int* zl = nullptr;             // band table of the sphere, then of the whole half spectrum (n/2 + 1 ints each)
+    const int* zl = nullptr;       // band table of the sphere, then of the whole half spectrum (n/2 + 1 ints
+                                   // each), behind the twiddles
     int xl = 0;                    // largest kx index inside the sphere
     int outside = 0;               // 1: v0 may hold modes outside the sphere (put, not projected since)
     double* d_famp = nullptr;      // per-stage band amplitude (fixed energy-injection forcing)
@@ -61,8 +62,9 @@ struct bfpsh_ctx {
     double* d_tab = nullptr;
     std::vector<int64_t> idx;
     std::vector<int64_t> order;    // slots in global-index order (set by particles_put)
-    uint32_t* d_rank = nullptr;    // rank of each slot in global-index order
-    double* d_samp = nullptr;      // sampling output, 2 x np x 9 doubles (raw, ranked)
+    uint32_t* d_order = nullptr;   // the same on the device
+    double* d_samp = nullptr;      // sampling output, np x 9 doubles in slot order
+    bool pool_user = false;        // counted among the users of the pinned transfer slots
     // standalone fields (field<rnumber, HIP, fc>): device buffer + ncomp per id
     std::vector<void*> fields;
     std::vector<int> field_nc;
@@ -248,6 +250,15 @@ void pass_wisdom_store(const std::string& key, const PassWisdom& w);
 
 int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, double dkz, int precision,
                int dealias, int device, hipStream_t stream, void* slab);
+
+// Host copies (transfer.hip): a whole field of nc planes in the host layout,
+// and the tracer rows [np][nc] in global-index order.  They wait for the copy.
+int bfpsh_field_to_host(bfpsh_ctx* ctx, bool real, int nc, const void* planes, void* host);
+int bfpsh_field_from_host(bfpsh_ctx* ctx, bool real, int nc, void* planes, const void* host);
+int bfpsh_rows_to_host(bfpsh_ctx* ctx, const double* rows, int nc, double* host);
+// a context begins / ceases to use the process's pinned transfer slots
+void bfpsh_transfer_open();
+void bfpsh_transfer_close();
 
 // tracer loop and sampling (particles.hip), dispatched on precision and
 // neighbour count
