@@ -1107,7 +1107,6 @@ int bfpsh_ensemble_create(bfpsh_ensemble** out, int nboxes, const int* sizes, in
             if (r) return efail(e, r, ctx ? ctx->err : "box creation failed");
             ctx->d_famp = c.d_famp + 3 * j;  // shared with the batch table (not freed by the box)
             ctx->force_coop = true;
-            ctx->sort_every = 16;
             // the first step's upload always differs from this placeholder
             c.sp[j].nu = -1.0;
         }

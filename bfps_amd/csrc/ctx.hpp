@@ -70,14 +70,15 @@ struct bfpsh_ctx {
     std::vector<int> field_nc;
     std::vector<char> field_real;  // 1 when the field holds real-space data
     // spatial ordering of the tracers (a permutation, data stays in place)
-    uint32_t* d_keys = nullptr;    // 2 x np
-    uint32_t* d_perm = nullptr;    // 2 x np
+    uint32_t* d_keys = nullptr;    // bucket of each tracer and its rank there (2 x np), and d_perm
+    uint32_t* d_perm = nullptr;    // the permutation (np, in the d_keys buffer)
     void* d_sort_tmp = nullptr;
     size_t sort_tmp_bytes = 0;
     double* d_crec = nullptr;      // column walk: per tracer in-cell fractions (3) + packed cells (np x 4)
-    uint32_t* d_bstart = nullptr;  // per-brick [start, end) (2 x nbricks)
-    int64_t nbricks = 0;
-    int sort_every = 1;            // re-sort period in tracer steps
+    uint32_t* d_bstart = nullptr;  // first place of each bucket (nbuckets + 1), then the counts or ends
+    uint32_t* d_bend = nullptr;    // end of each bucket, in the same buffer
+    int64_t nbuckets = 0;
+    int sort_every = 16;           // tracer steps between two permutations of the gather form
     int sort_age = 1 << 30;        // steps since the last sort
     // strided-pass tile shapes: index into pass_shapes<T, N>() per pass kind
     // (BFPSH_PASS_*), chosen by the pass autotuner (bfpsh_set_plan_rigor)

@@ -5,12 +5,14 @@
 // particles_adams_bashforth::move_particles (particles_adams_bashforth.hpp:18-133),
 // particles_system::completeLoop (particles_system.hpp:173-217).
 //
-// Tracer data stay in index order in device memory.  Each loop first sorts a
-// permutation of the tracers by the Morton code of their 4^3-cell
-// micro-brick (the reference buckets by z-slab for the same reason,
-// particles_utils.hpp:106-165), so consecutive threads interpolate nearby
-// tracers and share stencil rows in L1/L2; blocks are mapped so that each
-// XCD receives a contiguous run of the sorted order.
+// Tracer data stay in index order in device memory.  A permutation of the
+// tracers, bucketed by brick, by column and y step, or by the Morton code of
+// their micro-brick (the reference buckets by z-slab for the same reason,
+// particles_utils.hpp:106-165), makes consecutive threads interpolate nearby
+// tracers and share stencil rows; blocks are mapped so that each XCD receives
+// a contiguous run of the sorted order.  Bricks and columns need the buckets
+// of every step; the gather takes any order, so its permutation (of locality
+// only) is renewed every sort_every steps.
 //
 // Per tracer and axis: cell = floor(pos / h) mod N, x = position in the cell
 // in [0, 1); weights beta_j(x), j = 0..2n+1, for nodes cell-n .. cell+n+1
@@ -59,15 +61,45 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v) {
     return v;
 }
 
+// Bucketing of up to kCountSort tracers: a key kernel counts the tracers of
+// each bucket and keeps each one's rank among them, a scan gives the buckets'
+// first places, k_place writes the permutation.  That is five launches, where
+// a radix sort of the keys takes 10 at 10^5 tracers and 21 at 2^20 (5 to 7 us
+// each: 54 against 13 us at 10^5 in 128^3, 176 against 72 us at 2^20).  The
+// order within a bucket is that of the atomics; no result depends on it.  Above,
+// the returning atomics cost more than the sort, whose one-sweep form needs four
+// launches (2^22 tracers: 258 us by counting, 155 us by sorting).
+constexpr int64_t kCountSort = int64_t(1) << 20;
+__global__ void __launch_bounds__(256)
+k_place(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ rank, const uint32_t* __restrict__ start,
+        uint32_t* __restrict__ perm, int64_t np) {
+    const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (p < np) perm[start[keys[p]] + rank[p]] = uint32_t(p);
+}
+
+// [start, end) of each bucket in the sorted order (buckets without tracers keep
+// the zero fill)
+__global__ void k_bounds(const uint32_t* __restrict__ skeys, int64_t np, uint32_t* __restrict__ start,
+                         uint32_t* __restrict__ end) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const uint32_t k = skeys[i];
+    if (i == 0 || skeys[i - 1] != k) start[k] = uint32_t(i);
+    if (i == np - 1 || skeys[i + 1] != k) end[k] = uint32_t(i + 1);
+}
+
+// Keys of the buckets and, without counts, the tracers' numbers for the sort
+// in the place of their ranks
 __global__ void k_part_keys(const double* __restrict__ pos, int64_t np, PartGeomD pg, int shift,
-                            uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                            uint32_t* __restrict__ keys, uint32_t* __restrict__ rank, uint32_t* __restrict__ count) {
     const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (p >= np) return;
     const int cx = cell_of(pos[p * 3 + 0], pg.h[0], pg.n) >> shift;
     const int cy = cell_of(pos[p * 3 + 1], pg.h[1], pg.n) >> shift;
     const int cz = cell_of(pos[p * 3 + 2], pg.h[2], pg.n) >> shift;
-    keys[p] = spread3(cx) | (spread3(cy) << 1) | (spread3(cz) << 2);
-    vals[p] = uint32_t(p);
+    const uint32_t k = spread3(cx) | (spread3(cy) << 1) | (spread3(cz) << 2);
+    keys[p] = k;
+    rank[p] = count ? atomicAdd(&count[k], 1u) : uint32_t(p);
 }
 
 // logical block index so that XCD k (blocks dispatched round-robin over 8
@@ -451,25 +483,16 @@ __device__ __forceinline__ uint32_t brick_of(uint32_t logical, uint32_t nbx, uin
 }
 
 __global__ void k_brick_keys(const double* __restrict__ pos, int64_t np, PartGeomD pg, int kx, int ky, int kz,
-                             int nbx, int nby, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                             int nbx, int nby, uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                             uint32_t* __restrict__ count) {
     const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (p >= np) return;
     const int cx = cell_of(pos[p * 3 + 0], pg.h[0], pg.n) / kx;
     const int cy = cell_of(pos[p * 3 + 1], pg.h[1], pg.n) / ky;
     const int cz = cell_of(pos[p * 3 + 2], pg.h[2], pg.n) / kz;
-    keys[p] = uint32_t((cz * nby + cy) * nbx + cx);
-    vals[p] = uint32_t(p);
-}
-
-// [bstart, bend) of each brick in the sorted order (bricks without tracers
-// keep the zero fill)
-__global__ void k_brick_bounds(const uint32_t* __restrict__ skeys, int64_t np, uint32_t* __restrict__ bstart,
-                               uint32_t* __restrict__ bend) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= np) return;
-    const uint32_t k = skeys[i];
-    if (i == 0 || skeys[i - 1] != k) bstart[k] = uint32_t(i);
-    if (i == np - 1 || skeys[i + 1] != k) bend[k] = uint32_t(i + 1);
+    const uint32_t k = uint32_t((cz * nby + cy) * nbx + cx);
+    keys[p] = k;
+    rank[p] = count ? atomicAdd(&count[k], 1u) : uint32_t(p);
 }
 
 // y weights of the lane rows and all z weights, spread within each 16-lane
@@ -955,8 +978,8 @@ struct ColCfg {
 // record for the walk: in-cell fractions (get_norm_pos_in_cell /
 // pbc_field_layer, as k_brick's prologue) and the cell, 10 bits per axis
 __global__ void k_col_keys(const double* __restrict__ pos, int64_t np, PartGeomD pg, int kx, int ky, int kz,
-                           int ncx, int nys, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-                           double* __restrict__ rec) {
+                           int ncx, int nys, uint32_t* __restrict__ keys, uint32_t* __restrict__ rank,
+                           uint32_t* __restrict__ count, double* __restrict__ rec) {
     const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (p >= np) return;
     int cell[3];
@@ -970,8 +993,9 @@ __global__ void k_col_keys(const double* __restrict__ pos, int64_t np, PartGeomD
         fr[d] = (inbox - ci * pg.h[d]) / pg.h[d];
         cell[d] = cell_of(sp, pg.h[d], pg.n);
     }
-    keys[p] = uint32_t(((cell[2] / kz) * ncx + cell[0] / kx) * nys + cell[1] / ky);
-    vals[p] = uint32_t(p);
+    const uint32_t k = uint32_t(((cell[2] / kz) * ncx + cell[0] / kx) * nys + cell[1] / ky);
+    keys[p] = k;
+    rank[p] = count ? atomicAdd(&count[k], 1u) : uint32_t(p);
     double4 r;
     r.x = fr[0];
     r.y = fr[1];
@@ -1294,78 +1318,99 @@ unsigned blocks_for(int64_t np, int lp) {
     return unsigned(nb);
 }
 
-int ensure_sort(bfpsh_ctx* ctx) {
-    if (ctx->d_keys) return BFPSH_OK;
+// buffers of the bucketing into nk buckets: keys and ranks (sorting: keys and
+// numbers, then both sorted), the permutation, first places and counts (ends)
+int ensure_buckets(bfpsh_ctx* ctx, int64_t nk) {
     const int64_t np = ctx->np;
-    HIPCHK(hipMalloc((void**)&ctx->d_keys, 2 * np * sizeof(uint32_t)));
-    HIPCHK(hipMalloc((void**)&ctx->d_perm, 2 * np * sizeof(uint32_t)));
+    const bool sort = np > kCountSort;
+    if (!ctx->d_keys) {
+        HIPCHK(hipMalloc((void**)&ctx->d_keys, (sort ? 4 : 3) * np * sizeof(uint32_t)));
+        ctx->d_perm = ctx->d_keys + (sort ? 3 : 2) * np;
+        ctx->bytes += (sort ? 4 : 3) * np * sizeof(uint32_t);
+        ctx->sort_age = 1 << 30;
+    }
+    if (ctx->d_bstart && ctx->nbuckets >= nk) return BFPSH_OK;
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (void* p : {(void*)ctx->d_bstart, ctx->d_sort_tmp})
+        if (p) HIPCHK(hipFree(p));
+    ctx->d_bstart = nullptr;
+    ctx->d_sort_tmp = nullptr;
+    if (ctx->nbuckets) ctx->bytes -= 2 * (ctx->nbuckets + 1) * sizeof(uint32_t) + ctx->sort_tmp_bytes;
+    ctx->nbuckets = 0;
     size_t tmp = 0;
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, ctx->d_keys, ctx->d_keys + np, ctx->d_perm,
-                                              ctx->d_perm + np, int(np), 0, 30, ctx->stream));
-    HIPCHK(hipMalloc(&ctx->d_sort_tmp, tmp));
+    uint32_t* u = nullptr;
+    if (sort)
+        HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, u, u, u, u, int(np), 0, 30, ctx->stream));
+    else
+        HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, u, u, int(nk + 1), ctx->stream));
+    HIPCHK(hipMalloc((void**)&ctx->d_bstart, 2 * (nk + 1) * sizeof(uint32_t)));
+    HIPCHK(hipMalloc(&ctx->d_sort_tmp, std::max<size_t>(tmp, 16)));
     ctx->sort_tmp_bytes = tmp;
-    ctx->bytes += 4 * np * sizeof(uint32_t) + tmp;
-    ctx->sort_age = 1 << 30;
+    ctx->nbuckets = nk;
+    ctx->bytes += 2 * (nk + 1) * sizeof(uint32_t) + tmp;
     return BFPSH_OK;
 }
 
-// sorted permutation in d_perm + np
-int sort_tracers(bfpsh_ctx* ctx) {
-    int r = ensure_sort(ctx);
+// Bucket the tracers into nk buckets: keys(keys, ranks, counts) launches the
+// key kernel; the permutation ends in d_perm, bucket k's places in
+// [d_bstart[k], d_bend[k])
+template <class K>
+int bucket_tracers(bfpsh_ctx* ctx, int64_t nk, K&& keys) {
+    int r = ensure_buckets(ctx, nk);
     if (r) return r;
     const int64_t np = ctx->np;
-    const int shift = ctx->n >= 64 ? 2 : 0;
-    int nbits = 0;
-    while ((1 << nbits) < (ctx->n >> shift)) nbits++;
-    nbits *= 3;
-    LAUNCH("part_keys", (k_part_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(
-                            ctx->d_pos, np, pgeom_d(ctx), shift, ctx->d_keys, ctx->d_perm)));
+    const unsigned grid = unsigned((np + 255) / 256);
+    uint32_t* second = ctx->d_bstart + ctx->nbuckets + 1;
     size_t tmp = ctx->sort_tmp_bytes;
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(ctx->d_sort_tmp, tmp, ctx->d_keys, ctx->d_keys + np, ctx->d_perm,
-                                              ctx->d_perm + np, int(np), 0, std::max(nbits, 1), ctx->stream));
+    if (np > kCountSort) {
+        ctx->d_bend = second;
+        HIPCHK(hipMemsetAsync(ctx->d_bstart, 0, 2 * (ctx->nbuckets + 1) * sizeof(uint32_t), ctx->stream));
+        LAUNCH("part_keys", keys(ctx->d_keys, ctx->d_keys + np, (uint32_t*)nullptr));
+        int nbits = 1;
+        while ((int64_t(1) << nbits) < nk) nbits++;
+        uint32_t* sorted = ctx->d_keys + 2 * np;
+        HIPCHK(hipcub::DeviceRadixSort::SortPairs(ctx->d_sort_tmp, tmp, ctx->d_keys, sorted, ctx->d_keys + np,
+                                                  ctx->d_perm, int(np), 0, nbits, ctx->stream));
+        LAUNCH("part_bounds", (k_bounds<<<grid, 256, 0, ctx->stream>>>(sorted, np, ctx->d_bstart, second)));
+    } else {
+        ctx->d_bend = ctx->d_bstart + 1;
+        HIPCHK(hipMemsetAsync(second, 0, (nk + 1) * sizeof(uint32_t), ctx->stream));
+        LAUNCH("part_keys", keys(ctx->d_keys, ctx->d_keys + np, second));
+        HIPCHK(hipcub::DeviceScan::ExclusiveSum(ctx->d_sort_tmp, tmp, second, ctx->d_bstart, int(nk + 1), ctx->stream));
+        LAUNCH("part_place", (k_place<<<grid, 256, 0, ctx->stream>>>(ctx->d_keys, ctx->d_keys + np, ctx->d_bstart,
+                                                                     ctx->d_perm, np)));
+    }
     ctx->sort_age = 0;
     return BFPSH_OK;
 }
 
-template <typename T, int NB>
-int ensure_bricks(bfpsh_ctx* ctx, int64_t nb) {
-    if (ctx->d_bstart && ctx->nbricks == nb) return BFPSH_OK;
-    if (ctx->d_bstart) {
-        HIPCHK(hipStreamSynchronize(ctx->stream));
-        HIPCHK(hipFree(ctx->d_bstart));
-        ctx->d_bstart = nullptr;
+// by the Morton code of micro-bricks of 4^3 cells (1 below 64^3), larger ones
+// where there would be more than a few micro-bricks a tracer
+int sort_tracers(bfpsh_ctx* ctx) {
+    const int64_t np = ctx->np;
+    int shift = ctx->n >= 64 ? 2 : 0, nbits = 0;
+    while ((1 << nbits) < ((ctx->n - 1) >> shift) + 1) nbits++;
+    while (nbits > 0 && ((int64_t(1) << (3 * nbits)) > std::max<int64_t>(4 * np, 512) || 3 * nbits > 21)) {
+        nbits--;
+        shift++;
     }
-    HIPCHK(hipMalloc((void**)&ctx->d_bstart, 2 * nb * sizeof(uint32_t)));
-    ctx->nbricks = nb;
-    ctx->bytes += 2 * nb * sizeof(uint32_t);
-    return BFPSH_OK;
+    return bucket_tracers(ctx, int64_t(1) << (3 * nbits), [&](uint32_t* keys, uint32_t* rank, uint32_t* count) {
+        k_part_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(ctx->d_pos, np, pgeom_d(ctx), shift, keys, rank,
+                                                                         count);
+    });
 }
 
-// bucket the tracers by brick: sorted permutation in d_perm + np, per-brick
-// ranges in d_bstart[0..nb), d_bstart[nb..2nb)
+// by brick
 template <typename T, int NB>
 int sort_bricks(bfpsh_ctx* ctx) {
     using BC = BrickCfg<T, NB>;
-    int r = ensure_sort(ctx);
-    if (r) return r;
     const int n = ctx->n;
     const int nbx = n / BC::KX, nby = n / BC::KY, nbz = n / BC::KZ;
-    const int64_t nb = int64_t(nbx) * nby * nbz;
-    r = ensure_bricks<T, NB>(ctx, nb);
-    if (r) return r;
     const int64_t np = ctx->np;
-    int nbits = 1;
-    while ((int64_t(1) << nbits) < nb) nbits++;
-    HIPCHK(hipMemsetAsync(ctx->d_bstart, 0, 2 * nb * sizeof(uint32_t), ctx->stream));
-    LAUNCH("part_keys", (k_brick_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(
-                            ctx->d_pos, np, pgeom_d(ctx), BC::KX, BC::KY, BC::KZ, nbx, nby, ctx->d_keys, ctx->d_perm)));
-    size_t tmp = ctx->sort_tmp_bytes;
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(ctx->d_sort_tmp, tmp, ctx->d_keys, ctx->d_keys + np, ctx->d_perm,
-                                              ctx->d_perm + np, int(np), 0, nbits, ctx->stream));
-    LAUNCH("part_bounds", (k_brick_bounds<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(
-                              ctx->d_keys + np, np, ctx->d_bstart, ctx->d_bstart + nb)));
-    ctx->sort_age = 0;
-    return BFPSH_OK;
+    return bucket_tracers(ctx, int64_t(nbx) * nby * nbz, [&](uint32_t* keys, uint32_t* rank, uint32_t* count) {
+        k_brick_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(ctx->d_pos, np, pgeom_d(ctx), BC::KX, BC::KY,
+                                                                          BC::KZ, nbx, nby, keys, rank, count);
+    });
 }
 
 template <typename T, int NB, int NC, int MODE>
@@ -1383,8 +1428,8 @@ int launch_brick(bfpsh_ctx* ctx, const void* f, double* d_out, double dt, int or
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
     const unsigned grid = unsigned(std::max<int64_t>(1, std::min<int64_t>(nb, ncu)));
     LAUNCH(name, (kern<<<grid, BC::NT, lds, ctx->stream>>>(
-                     (const T*)f, ctx->d_pos, ctx->d_rhs, d_out, ctx->d_perm + ctx->np, ctx->d_bstart,
-                     ctx->d_bstart + nb, nbx, nby, ctx->np, ctx->nsteps, ctx->head, order, ctx->add_head ? 1 : 0, dt,
+                     (const T*)f, ctx->d_pos, ctx->d_rhs, d_out, ctx->d_perm, ctx->d_bstart,
+                     ctx->d_bend, nbx, nby, ctx->np, ctx->nsteps, ctx->head, order, ctx->add_head ? 1 : 0, dt,
                      ctx->d_tab, ctx->deg, pgeom_d(ctx))));
     return BFPSH_OK;
 }
@@ -1416,40 +1461,25 @@ bool col_geom(const bfpsh_ctx* ctx, ColGeom& g) {
     return g.sps <= CC::MAXS;
 }
 
-// bucket the tracers by (column, y step): sorted permutation in d_perm + np,
-// per-key ranges in d_bstart[0..nk), d_bstart[nk..2nk)
+// by (column, y step)
 template <typename T, int NB>
 int sort_cols(bfpsh_ctx* ctx, const ColGeom& g) {
     using CC = ColCfg<T, NB>;
-    int r = ensure_sort(ctx);
-    if (r) return r;
-    const int64_t nk = int64_t(g.ncols) * g.nys;
-    r = ensure_bricks<T, NB>(ctx, nk);
-    if (r) return r;
     const int64_t np = ctx->np;
     if (!ctx->d_crec) {
         HIPCHK(hipMalloc((void**)&ctx->d_crec, size_t(np) * 4 * sizeof(double)));
         ctx->bytes += size_t(np) * 4 * sizeof(double);
     }
-    int nbits = 1;
-    while ((int64_t(1) << nbits) < nk) nbits++;
-    HIPCHK(hipMemsetAsync(ctx->d_bstart, 0, 2 * nk * sizeof(uint32_t), ctx->stream));
-    LAUNCH("part_keys", (k_col_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(
-                            ctx->d_pos, np, pgeom_d(ctx), CC::KX, CC::KY, CC::KZ, g.ncx, g.nys, ctx->d_keys,
-                            ctx->d_perm, ctx->d_crec)));
-    size_t tmp = ctx->sort_tmp_bytes;
-    HIPCHK(hipcub::DeviceRadixSort::SortPairs(ctx->d_sort_tmp, tmp, ctx->d_keys, ctx->d_keys + np, ctx->d_perm,
-                                              ctx->d_perm + np, int(np), 0, nbits, ctx->stream));
-    LAUNCH("part_bounds", (k_brick_bounds<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(
-                              ctx->d_keys + np, np, ctx->d_bstart, ctx->d_bstart + nk)));
-    ctx->sort_age = 0;
-    return BFPSH_OK;
+    return bucket_tracers(ctx, int64_t(g.ncols) * g.nys, [&](uint32_t* keys, uint32_t* rank, uint32_t* count) {
+        k_col_keys<<<unsigned((np + 255) / 256), 256, 0, ctx->stream>>>(ctx->d_pos, np, pgeom_d(ctx), CC::KX, CC::KY,
+                                                                        CC::KZ, g.ncx, g.nys, keys, rank, count,
+                                                                        ctx->d_crec);
+    });
 }
 
 template <typename T, int NB, int NC, int MODE>
 int launch_col(bfpsh_ctx* ctx, const ColGeom& g, const void* f, double* d_out, const char* name) {
     using CC = ColCfg<T, NB>;
-    const int64_t nk = int64_t(g.ncols) * g.nys;
     auto kern = k_column<T, NB, NC, MODE>;
     HIPCHK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(CC::LDS)));
     int ncu = 0;
@@ -1457,7 +1487,7 @@ int launch_col(bfpsh_ctx* ctx, const ColGeom& g, const void* f, double* d_out, c
     // one workgroup per CU, persistent over its work items
     const unsigned grid = unsigned(std::max(1, std::min(g.nwork, ncu)));
     LAUNCH(name, (kern<<<grid, CC::NT, CC::LDS, ctx->stream>>>(
-                     (const T*)f, ctx->d_crec, d_out, ctx->d_perm + ctx->np, ctx->d_bstart, ctx->d_bstart + nk, g.ncx,
+                     (const T*)f, ctx->d_crec, d_out, ctx->d_perm, ctx->d_bstart, ctx->d_bend, g.ncx,
                      g.nys, g.ncols, g.sps, g.nwork, ctx->np, ctx->head, ctx->add_head ? 1 : 0, ctx->d_tab, ctx->deg,
                      pgeom_d(ctx))));
     return BFPSH_OK;
@@ -1503,7 +1533,7 @@ int sample_form(bfpsh_ctx* ctx, int form, const void* f, int nc, double* d_out) 
             return launch_brick<T, NB, 9, 1>(ctx, f, d_out, 0.0, 0, "sample9");
         }
     }
-    {
+    if (ctx->sort_age >= ctx->sort_every) {
         int r = sort_tracers(ctx);
         if (r) return r;
     }
@@ -1512,18 +1542,18 @@ int sample_form(bfpsh_ctx* ctx, int form, const void* f, int nc, double* d_out) 
         if (nc == 1) {
             LAUNCH("sample1_gather", (k_sample<T, NB, 1><<<blocks_for(ctx->np, Lanes<NB>::LP), kThreads, lds,
                                                           ctx->stream>>>((const T*)f, ctx->d_pos, d_out,
-                                                                         ctx->d_perm + ctx->np, ctx->np, ctx->d_tab,
+                                                                         ctx->d_perm, ctx->np, ctx->d_tab,
                                                                          ctx->deg, pgeom_d(ctx))));
             return BFPSH_OK;
         }
     if (nc == 3)
         LAUNCH("sample_gather", (k_sample<T, NB, 3><<<blocks_for(ctx->np, Lanes<NB>::LP), kThreads, lds, ctx->stream>>>(
-                                    (const T*)f, ctx->d_pos, d_out, ctx->d_perm + ctx->np, ctx->np, ctx->d_tab, ctx->deg,
+                                    (const T*)f, ctx->d_pos, d_out, ctx->d_perm, ctx->np, ctx->d_tab, ctx->deg,
                                     pgeom_d(ctx))));
     else
         LAUNCH("sample9_gather", (k_sample<T, NB, 9><<<blocks_for(ctx->np, Lanes<NB>::LP), kThreads, lds,
                                                       ctx->stream>>>((const T*)f, ctx->d_pos, d_out,
-                                                                     ctx->d_perm + ctx->np, ctx->np, ctx->d_tab,
+                                                                     ctx->d_perm, ctx->np, ctx->d_tab,
                                                                      ctx->deg, pgeom_d(ctx))));
     return BFPSH_OK;
 }
@@ -1559,7 +1589,7 @@ int loop_form(bfpsh_ctx* ctx, int form, const void* u, double dt, int order) {
     }
     const size_t lds = size_t(2 * NB + 2) * (ctx->deg + 1) * sizeof(double);
     LAUNCH("interp_ab_gather", (k_interp_ab<T, NB><<<blocks_for(ctx->np, Lanes<NB>::LP), kThreads, lds, ctx->stream>>>(
-                                   (const T*)u, ctx->d_pos, ctx->d_rhs, ctx->d_perm + ctx->np, ctx->np,
+                                   (const T*)u, ctx->d_pos, ctx->d_rhs, ctx->d_perm, ctx->np,
                                    ctx->nsteps, ctx->head, order, ctx->add_head ? 1 : 0, dt, ctx->d_tab, ctx->deg,
                                    pgeom_d(ctx))));
     return BFPSH_OK;
@@ -1624,7 +1654,7 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
         auto fresh = [&]() -> int {
             if (hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
                 return BFPSH_EHIP;
-            ctx->sort_age = 1 << 30;  // every form sorts, as in a step
+            ctx->sort_age = 1 << 30;  // bricks and columns sort, as in a step
             return BFPSH_OK;
         };
         double tbest = 1e300, tfirst = 0.0;
@@ -1633,6 +1663,9 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
             r = fresh();
             if (r == BFPSH_OK) r = loop_form<T, NB>(ctx, cand[i], u, 0.0, ctx->nsteps);  // warm-up
             if (r == BFPSH_OK) r = fresh();
+            // (the gather renews its permutation every sort_every steps: it
+            // is timed on the one of its warm-up)
+            if (cand[i] == FORM_GATHER && ctx->sort_every > 1) ctx->sort_age = 0;
             if (r == BFPSH_OK && hipEventRecord(a, ctx->stream) != hipSuccess) r = BFPSH_EHIP;
             if (r == BFPSH_OK) r = loop_form<T, NB>(ctx, cand[i], u, 0.0, ctx->nsteps);
             float ms = 0.f;
@@ -1745,7 +1778,7 @@ int prepare_group(const std::vector<bfpsh_ctx*>& boxes, const std::vector<double
         b.f = c->ru;
         b.pos = c->d_pos;
         b.rhs = c->d_rhs;
-        b.perm = c->d_perm + c->np;
+        b.perm = c->d_perm;
         b.tab = c->d_tab;
         b.np = c->np;
         b.pg = pgeom_d(c);
@@ -1904,11 +1937,11 @@ void bfpsh_part_batch_free(PartBatch& pb) {
 }
 
 int bfpsh_part_release(bfpsh_ctx* ctx) {
-    for (void* p : {(void*)ctx->d_keys, (void*)ctx->d_perm, ctx->d_sort_tmp, (void*)ctx->d_bstart, (void*)ctx->d_crec})
+    for (void* p : {(void*)ctx->d_keys, ctx->d_sort_tmp, (void*)ctx->d_bstart, (void*)ctx->d_crec})
         if (p) (void)hipFree(p);
     ctx->d_crec = nullptr;
-    ctx->d_bstart = nullptr;
-    ctx->nbricks = 0;
+    ctx->d_bstart = ctx->d_bend = nullptr;
+    ctx->nbuckets = 0;
     ctx->d_keys = nullptr;
     ctx->d_perm = nullptr;
     ctx->d_sort_tmp = nullptr;
