@@ -110,30 +110,6 @@ __device__ __forceinline__ int64_t xcd_block() {
     return (b % 8) * nb8 + b / 8;
 }
 
-template <int NB>
-__device__ __forceinline__ void setup_axis(double s, const double* __restrict__ tab, int deg, double width, double h,
-                                           int n, double (&bw)[2 * NB + 2], int (&idx)[2 * NB + 2]) {
-    constexpr int W = 2 * NB + 2;
-    // get_norm_pos_in_cell (particles_field_computer.hpp:55-63)
-    const double rep = floor(s / width);
-    const double inbox = s - rep * width;
-    const double ci = floor(inbox / h);
-    const double xr = (inbox - ci * h) / h;
-#pragma unroll
-    for (int j = 0; j < W; j++) {
-        double acc = 0.0;
-        for (int q = deg; q >= 0; q--) acc = acc * xr + tab[j * (deg + 1) + q];
-        bw[j] = acc;
-    }
-    const int c = cell_of(s, h, n);
-#pragma unroll
-    for (int j = 0; j < W; j++) {
-        int v = c - NB + j;
-        v = v < 0 ? v + n : (v >= n ? v - n : v);
-        idx[j] = v;
-    }
-}
-
 // Lanes per tracer: the W = 2n+2 stencil columns along x are spread over LP
 // lanes (the power of two from 4 to 32 that holds W), so one wavefront load
 // instruction reads 64/LP contiguous row segments instead of 64 scattered
@@ -143,55 +119,108 @@ template <int NB> struct Lanes {
     static constexpr int LP = W <= 4 ? 4 : (W <= 8 ? 8 : (W <= 16 ? 16 : 32));
 };
 
-// sum over the stencil of one tracer, computed by the LP lanes of its group;
-// lane jx < W holds column jx.  Result valid in every lane of the group.
+// LDS of one lane group: y and z weights, in-cell fractions, cells
+template <int NB> struct GroupLds {
+    static constexpr int W = 2 * NB + 2;
+    static constexpr int DOUBLES = 2 * W + 3 + 2;  // (3 ints in the last 2)
+    static constexpr int TOTAL = DOUBLES * (256 / Lanes<NB>::LP);
+};
+
+// Sum over the stencil of one tracer at xp[0..2], computed by the LP lanes of
+// its group; lane jx < W holds column jx.  Result valid in every lane of the
+// group.  Lane a < 3 locates the tracer on axis a, then lane j evaluates
+// weight j on the three axes; the others read them from the group's LDS wl.
+// (Every lane locating the tracer and evaluating all y and z weights for
+// itself took most of the time: 10^5 tracers n2 at 128^3, 77 us a loop.)  A
+// group lies inside one wave, so wave-level ordering is enough.
 template <typename T, int NB, int NC>
-__device__ __forceinline__ void gather_coop(const T* __restrict__ f, int n, const double* x,
-                                            const double* __restrict__ tab, int deg, const PartGeomD& pg,
-                                            int jx, double (&acc)[NC]) {
+__device__ __forceinline__ void gather_coop(const T* __restrict__ f, int n, const double* xp,
+                                            const double* __restrict__ tab, int deg, const PartGeomD& pg, int jx,
+                                            double* wl, double (&acc)[NC]) {
     constexpr int W = 2 * NB + 2;
     constexpr int LP = Lanes<NB>::LP;
-    double by[W], bz[W];
-    int iy[W], iz[W];
-    setup_axis<NB>(x[1], tab, deg, pg.width[1], pg.h[1], n, by, iy);
-    setup_axis<NB>(x[2], tab, deg, pg.width[2], pg.h[2], n, bz, iz);
-    // this lane's x column
-    double bxl = 0.0;
-    int ixl = 0;
-    {
-        const double s = x[0];
-        const double rep = floor(s / pg.width[0]);
-        const double inbox = s - rep * pg.width[0];
-        const double ci = floor(inbox / pg.h[0]);
-        const double xr = (inbox - ci * pg.h[0]) / pg.h[0];
-        const int jj = jx < W ? jx : 0;
-        double a = 0.0;
-        for (int q = deg; q >= 0; q--) a = a * xr + tab[jj * (deg + 1) + q];
-        bxl = jx < W ? a : 0.0;
-        int v = cell_of(s, pg.h[0], n) - NB + jj;
-        v = v < 0 ? v + n : (v >= n ? v - n : v);
-        ixl = v;
+    static_assert(LP >= 4 && LP >= W && 64 % LP == 0, "a lane for each axis and weight, groups inside a wave");
+    int* cl = reinterpret_cast<int*>(wl + 2 * W + 3);
+    if (jx < 3) {
+        // get_norm_pos_in_cell (particles_field_computer.hpp:55-63)
+        const double s = xp[jx];
+        const double width = jx == 0 ? pg.width[0] : (jx == 1 ? pg.width[1] : pg.width[2]);
+        const double h = jx == 0 ? pg.h[0] : (jx == 1 ? pg.h[1] : pg.h[2]);
+        const double rep = floor(s / width);
+        const double inbox = s - rep * width;
+        const double ci = floor(inbox / h);
+        wl[2 * W + jx] = (inbox - ci * h) / h;
+        cl[jx] = cell_of(s, h, n);
     }
+    wave_sync();
+    const double xr0 = wl[2 * W], xr1 = wl[2 * W + 1], xr2 = wl[2 * W + 2];
+    const int c0 = cl[0], c1 = cl[1], c2 = cl[2];
+    const int jj = jx < W ? jx : 0;
+    double w0 = 0.0, w1 = 0.0, w2 = 0.0;
+    for (int q = deg; q >= 0; q--) {
+        const double k = tab[jj * (deg + 1) + q];
+        w0 = fma(w0, xr0, k);
+        w1 = fma(w1, xr1, k);
+        w2 = fma(w2, xr2, k);
+    }
+    if (jx < W) {
+        wl[jx] = w1;
+        wl[W + jx] = w2;
+    }
+    wave_sync();
     // real planes 2 plane_size(n) reals apart, y rows 2 row_stride(n) apart
     const size_t ps = 2 * plane_size(n), ys = 2 * row_stride(n);
+    auto wrap = [n](int v) { return v < 0 ? v + n : (v >= n ? v - n : v); };
 #pragma unroll
     for (int c = 0; c < NC; c++) acc[c] = 0.0;
     if (jx < W) {
-        for (int jz = 0; jz < W; jz++) {
+        const T* col0 = f + wrap(c0 - NB + jj);
+        // the values of plane jz + 1 are requested before those of plane jz
+        // are summed, where two planes fit in registers
+        constexpr bool AHEAD = W * NC * int(sizeof(T)) <= 144;
+        T va[W][NC], vb[W][NC];
+        auto load = [&](int jz, T (&v)[W][NC]) {
+            const T* colz = col0 + size_t(wrap(c2 - NB + jz)) * n;
+#pragma unroll
+            for (int jy = 0; jy < W; jy++) {
+                const T* p = colz + size_t(wrap(c1 - NB + jy)) * ys;
+#pragma unroll
+                for (int c = 0; c < NC; c++) v[jy][c] = p[c * ps];
+            }
+        };
+        auto sum = [&](int jz, const T (&v)[W][NC]) {
             double col[NC];
 #pragma unroll
             for (int c = 0; c < NC; c++) col[c] = 0.0;
-#pragma unroll 2
+#pragma unroll
             for (int jy = 0; jy < W; jy++) {
-                const size_t pt = size_t(iy[jy]) * ys + size_t(iz[jz]) * n + ixl;
+                const double by = wl[jy];
 #pragma unroll
-                for (int c = 0; c < NC; c++) col[c] = fma(by[jy], double(f[c * ps + pt]), col[c]);
+                for (int c = 0; c < NC; c++) col[c] = fma(by, double(v[jy][c]), col[c]);
             }
+            const double bz = wl[W + jz];
 #pragma unroll
-            for (int c = 0; c < NC; c++) acc[c] = fma(bz[jz], col[c], acc[c]);
+            for (int c = 0; c < NC; c++) acc[c] = fma(bz, col[c], acc[c]);
+        };
+        if constexpr (AHEAD) {
+            static_assert(W % 2 == 0, "planes in pairs");
+            load(0, va);
+#pragma unroll 1
+            for (int jz = 0; jz < W; jz += 2) {
+                load(jz + 1, vb);
+                sum(jz, va);
+                if (jz + 2 < W) load(jz + 2, va);
+                sum(jz + 1, vb);
+            }
+        } else {
+#pragma unroll 1
+            for (int jz = 0; jz < W; jz++) {
+                load(jz, va);
+                sum(jz, va);
+            }
         }
 #pragma unroll
-        for (int c = 0; c < NC; c++) acc[c] *= bxl;
+        for (int c = 0; c < NC; c++) acc[c] *= w0;
     }
 #pragma unroll
     for (int c = 0; c < NC; c++) {
@@ -200,48 +229,46 @@ __device__ __forceinline__ void gather_coop(const T* __restrict__ f, int n, cons
     }
 }
 
+// Adams-Bashforth increment of one coordinate from the right-hand sides r[0]
+// (newest) .. r[order - 1] (particles_adams_bashforth.hpp:18-133)
+BFPSH_DEV double ab_increment(const double (&r)[6], int order, double dt) {
+    switch (order) {
+    case 1: return dt * r[0];
+    case 2: return dt * (3. * r[0] - r[1]) / 2.;
+    case 3: return dt * (23. * r[0] - 16. * r[1] + 5. * r[2]) / 12.;
+    case 4: return dt * (55. * r[0] - 59. * r[1] + 37. * r[2] - 9. * r[3]) / 24.;
+    case 5: return dt * (1901. * r[0] - 2774. * r[1] + 2616. * r[2] - 1274. * r[3] + 251. * r[4]) / 720.;
+    default: return dt * (4277. * r[0] - 7923. * r[1] + 9982. * r[2] - 7298. * r[3] + 2877. * r[4] - 475. * r[5]) / 1440.;
+    }
+}
+
 // One tracer of the Adams-Bashforth loop (MODE 0 of the brick kernel, for
 // the global-gather path): velocity at the tracer into the history head,
-// then the position update of order `order`.  t = rank of the tracer in the
-// sorted order, jx = lane in its group.
+// then the position update of order `order`, lane d < 3 of the group for
+// coordinate d.  t = rank of the tracer in the sorted order, jx = lane in its
+// group.
 template <typename T, int NB>
-__device__ __forceinline__ void interp_ab_one(const T* __restrict__ f, double* __restrict__ pos,
-                                              double* __restrict__ rhs, const uint32_t* __restrict__ perm,
-                                              int64_t np, int nsteps, int head, int order, int add_head, double dt,
-                                              const double* stab, int deg, const PartGeomD& pg, int64_t t, int jx) {
+__device__ __forceinline__ void interp_ab_one(const T* __restrict__ f, double* pos, double* __restrict__ rhs,
+                                              const uint32_t* __restrict__ perm, int64_t np, int nsteps, int head,
+                                              int order, int add_head, double dt, const double* stab, int deg,
+                                              const PartGeomD& pg, int64_t t, int jx, double* wl) {
     const int64_t p = perm[t];
-    double x[3] = {pos[p * 3 + 0], pos[p * 3 + 1], pos[p * 3 + 2]};
     double r0[3];
-    gather_coop<T, NB, 3>(f, pg.n, x, stab, deg, pg, jx, r0);
-    if (jx != 0) return;
-    double* h0 = rhs + size_t(head) * np * 3 + p * 3;
-    if (add_head) {
-        r0[0] += h0[0];
-        r0[1] += h0[1];
-        r0[2] += h0[2];
-    }
-    h0[0] = r0[0];
-    h0[1] = r0[1];
-    h0[2] = r0[2];
+    gather_coop<T, NB, 3>(f, pg.n, pos + p * 3, stab, deg, pg, jx, wl, r0);
+    if (jx >= 3) return;
+    const size_t at = size_t(p) * 3 + jx, slot = size_t(np) * 3;
+    double r[6];
+    r[0] = jx == 0 ? r0[0] : (jx == 1 ? r0[1] : r0[2]);
+    double* h0 = rhs + size_t(head) * slot + at;
+    if (add_head) r[0] += *h0;
+    *h0 = r[0];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        double r[6];
-        r[0] = r0[d];
-        for (int i = 1; i < order; i++) r[i] = rhs[size_t((head + i) % nsteps) * np * 3 + p * 3 + d];
-        double incr;
-        switch (order) {
-        case 1: incr = dt * r[0]; break;
-        case 2: incr = dt * (3. * r[0] - r[1]) / 2.; break;
-        case 3: incr = dt * (23. * r[0] - 16. * r[1] + 5. * r[2]) / 12.; break;
-        case 4: incr = dt * (55. * r[0] - 59. * r[1] + 37. * r[2] - 9. * r[3]) / 24.; break;
-        case 5: incr = dt * (1901. * r[0] - 2774. * r[1] + 2616. * r[2] - 1274. * r[3] + 251. * r[4]) / 720.; break;
-        default: incr = dt * (4277. * r[0] - 7923. * r[1] + 9982. * r[2] - 7298. * r[3] + 2877. * r[4] - 475. * r[5]) / 1440.; break;
-        }
-        x[d] += incr;
+    for (int i = 1; i < 6; i++) {
+        int s = head + i;
+        s = s >= nsteps ? s - nsteps : s;  // i < order <= nsteps
+        r[i] = i < order ? rhs[size_t(s) * slot + at] : 0.0;
     }
-    pos[p * 3 + 0] = x[0];
-    pos[p * 3 + 1] = x[1];
-    pos[p * 3 + 2] = x[2];
+    pos[at] += ab_increment(r, order, dt);
 }
 
 template <typename T, int NB>
@@ -251,13 +278,15 @@ k_interp_ab(const T* __restrict__ f, double* __restrict__ pos, double* __restric
             double dt, const double* __restrict__ tab, int deg, PartGeomD pg) {
     constexpr int LP = Lanes<NB>::LP;
     extern __shared__ double stab[];
+    __shared__ double wl[GroupLds<NB>::TOTAL];
     const int tabsize = (2 * NB + 2) * (deg + 1);  // derivative-0 block only
     for (int i = threadIdx.x; i < tabsize; i += blockDim.x) stab[i] = tab[i];
     __syncthreads();
     const int64_t t = (xcd_block() * blockDim.x + threadIdx.x) / LP;
     const int jx = threadIdx.x % LP;
     if (t >= np) return;  // whole lane groups exit together
-    interp_ab_one<T, NB>(f, pos, rhs, perm, np, nsteps, head, order, add_head, dt, stab, deg, pg, t, jx);
+    interp_ab_one<T, NB>(f, pos, rhs, perm, np, nsteps, head, order, add_head, dt, stab, deg, pg, t, jx,
+                         wl + threadIdx.x / LP * GroupLds<NB>::DOUBLES);
 }
 
 // The tracer loops of many boxes (an ensemble) in one launch: box b owns
@@ -305,6 +334,7 @@ __global__ void __launch_bounds__(256)
 k_interp_ab_multi(const TracerBox* __restrict__ boxes, const TracerDyn* __restrict__ dyn, int nboxes) {
     constexpr int LP = Lanes<NB>::LP;
     extern __shared__ double stab[];
+    __shared__ double wl[GroupLds<NB>::TOTAL];
     // the box of this workgroup: the last one starting at or before it
     int lo = 0, hi = nboxes - 1;
     while (lo < hi) {
@@ -320,10 +350,11 @@ k_interp_ab_multi(const TracerBox* __restrict__ boxes, const TracerDyn* __restri
     const int64_t t = (int64_t(blockIdx.x - bx.block0) * blockDim.x + threadIdx.x) / LP;
     const int jx = threadIdx.x % LP;
     if (t >= bx.np) return;  // whole lane groups exit together
-    const PartGeomD pg = bx.pg;
+    const PartGeomD& pg = bx.pg;
     const TracerDyn d = dyn[lo];
     interp_ab_one<T, NB>((const T*)bx.f, bx.pos, bx.rhs, bx.perm, bx.np, bx.nsteps, d.head,
-                         min(d.step_idx, bx.nsteps), d.add_head, bx.dt, stab, deg, pg, t, jx);
+                         min(d.step_idx, bx.nsteps), d.add_head, bx.dt, stab, deg, pg, t, jx,
+                         wl + threadIdx.x / LP * GroupLds<NB>::DOUBLES);
 }
 
 template <typename T, int NB, int NC>
@@ -332,6 +363,7 @@ k_sample(const T* __restrict__ f, const double* __restrict__ pos, double* __rest
          const uint32_t* __restrict__ perm, int64_t np, const double* __restrict__ tab, int deg, PartGeomD pg) {
     constexpr int LP = Lanes<NB>::LP;
     extern __shared__ double stab[];
+    __shared__ double wl[GroupLds<NB>::TOTAL];
     const int tabsize = (2 * NB + 2) * (deg + 1);
     for (int i = threadIdx.x; i < tabsize; i += blockDim.x) stab[i] = tab[i];
     __syncthreads();
@@ -339,9 +371,8 @@ k_sample(const T* __restrict__ f, const double* __restrict__ pos, double* __rest
     const int jx = threadIdx.x % LP;
     if (t >= np) return;
     const int64_t p = perm[t];
-    const double x[3] = {pos[p * 3 + 0], pos[p * 3 + 1], pos[p * 3 + 2]};
     double acc[NC];
-    gather_coop<T, NB, NC>(f, pg.n, x, stab, deg, pg, jx, acc);
+    gather_coop<T, NB, NC>(f, pg.n, pos + p * 3, stab, deg, pg, jx, wl + threadIdx.x / LP * GroupLds<NB>::DOUBLES, acc);
     if (jx != 0) return;
 #pragma unroll
     for (int c = 0; c < NC; c++) out[p * NC + c] = acc[c];
@@ -552,16 +583,7 @@ BFPSH_DEV void ab_move(double* __restrict__ pos, const double* __restrict__ rhs,
         double r[6];
         r[0] = r0[d];
         for (int i = 1; i < order; i++) r[i] = rhs[size_t((head + i) % nsteps) * np * 3 + p * 3 + d];
-        double incr;
-        switch (order) {
-        case 1: incr = dt * r[0]; break;
-        case 2: incr = dt * (3. * r[0] - r[1]) / 2.; break;
-        case 3: incr = dt * (23. * r[0] - 16. * r[1] + 5. * r[2]) / 12.; break;
-        case 4: incr = dt * (55. * r[0] - 59. * r[1] + 37. * r[2] - 9. * r[3]) / 24.; break;
-        case 5: incr = dt * (1901. * r[0] - 2774. * r[1] + 2616. * r[2] - 1274. * r[3] + 251. * r[4]) / 720.; break;
-        default: incr = dt * (4277. * r[0] - 7923. * r[1] + 9982. * r[2] - 7298. * r[3] + 2877. * r[4] - 475. * r[5]) / 1440.; break;
-        }
-        pos[p * 3 + d] = x[d] + incr;
+        pos[p * 3 + d] = x[d] + ab_increment(r, order, dt);
     }
 }
 
