@@ -69,8 +69,8 @@ int bfpsh_create(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky
  * each strided FFT pass kind is chosen among the compiled shapes:
  * ESTIMATE takes the shape the pass wisdom holds, else the built-in one;
  * MEASURE and PATIENT take the wisdom's shape when a search of at least
- * their rigor chose it, else time every compiled shape (3 launches each on
- * the work planes for MEASURE, 10 for PATIENT) and keep the fastest in
+ * their rigor chose it, else time every compiled shape (2 x 2 launches each
+ * on the work planes for MEASURE, 2 x 5 for PATIENT) and keep the fastest in
  * the wisdom.  Boxes below 256^3 have one shape.  At MEASURE and PATIENT
  * the first tracer loop or sample of a tracer set also times the velocity
  * loop of each applicable tracer kernel form (column walk, bricks, global
