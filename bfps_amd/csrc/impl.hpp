@@ -301,18 +301,20 @@ struct Impl {
                 LAUNCH("band_amplitude", (k_band_amplitude<T, N><<<1, 256, 0, ctx->stream>>>(
                                              src, bt.famp + (s - 1), g, bt.sp.famp, bt.sp.fk0, bt.sp.fk1, 0, nullptr, s)));
         }
-        {
+        if constexpr (Slab<T, N>::ok) {
+            LAUNCH("slab_cross", (k_slab_cross<T, N><<<dim3(N, nb), Slab<T, N>::NT, 0, ctx->stream>>>(
+                                     w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
+        } else {
             int r = pass(ctx, BFPSH_PASS_Z_INV, w, 6, "inv_z", bt.zl, nb, bs);
             if (r) return r;
-        }
-        if constexpr (RowsW<T, N>::ok && !BFPSH_ROWS_TILE)
-            LAUNCH("rows_cross", (k_rows_cross_w<T, N><<<dim3(N * N / 2 / RowsW<T, N>::RPB, nb), RowsW<T, N>::NT, 0,
-                                                         ctx->stream>>>(w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
-        else
-            LAUNCH("rows_cross", (k_rows_cross<T, N><<<dim3(N * N / 2 / CF::RP, nb), CF::NT_ROW, 0, ctx->stream>>>(
-                                      w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
-        {
-            int r = pass(ctx, BFPSH_PASS_Z_FWD, w, 3, "fwd_z", bt.zl, nb, bs);
+            if constexpr (RowsW<T, N>::ok)
+                LAUNCH("rows_cross", (k_rows_cross_w<T, N><<<dim3(N * N / 2 / RowsW<T, N>::RPB, nb), RowsW<T, N>::NT,
+                                                             0, ctx->stream>>>(w, ru, tw, bt.zl, T(double(N) * N * N),
+                                                                               bs)));
+            else
+                LAUNCH("rows_cross", (k_rows_cross<T, N><<<dim3(N * N / 2 / CF::RP, nb), CF::NT_ROW, 0, ctx->stream>>>(
+                                          w, ru, tw, bt.zl, T(double(N) * N * N), bs)));
+            r = pass(ctx, BFPSH_PASS_Z_FWD, w, 3, "fwd_z", bt.zl, nb, bs);
             if (r) return r;
         }
         const dim3 tiles3(NXH / CF::B_Y3, N, nb);

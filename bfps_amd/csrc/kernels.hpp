@@ -48,10 +48,6 @@
 #ifndef BFPSH_RW_PAD
 #define BFPSH_RW_PAD 4
 #endif
-// 1: x-axis rows through the LDS-tile FFT for every size (A/B switch)
-#ifndef BFPSH_ROWS_TILE
-#define BFPSH_ROWS_TILE 0
-#endif
 
 namespace bfpsh {
 
@@ -87,11 +83,14 @@ struct Cfg {
     static constexpr int BF = bcap(65536);
     // fused y passes (Biot-Savart, update): three components stay in
     // registers.  Small boxes run one short wave of workgroups, whose time is
-    // the code each one walks through once: fewer values per thread
+    // the code each one walks through once: fewer values per thread (FP32
+    // first stage at 16^3, 2 / 4 / 16 values: 11.1 / 13.7 / 22.5 us; 64^3,
+    // 4 / 8: 17.6 / 22.1 us; 256^3, 8 / 16: 218 / 239 us)
     static constexpr int efused() {
         if (N % 3 == 0) return 6;
-        if (N <= 64) return 4;
-        if (N == 128) return 8;
+        if (N <= 32) return 2;
+        if (N == 64) return 4;
+        if (N <= 256) return 8;
         return E;
     }
     // half the columns when the threads would exceed 512, to keep the
@@ -831,6 +830,178 @@ k_rows_cross_w(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __rest
             data[c * PS + rb + g + G * m] = mk<T>(T(0.5) * (Z.y + M.y), T(-0.5) * (Z.x - M.x));
         }
     }
+}
+
+// Small boxes: the middle of a stage in one launch.  A workgroup holds the
+// (z, x) slab of one y: inverse z pass, c2r x pass, cross product, r2c x pass
+// and forward z pass of k_pass, k_rows_cross and k_pass above, with the same
+// band.  At these sizes each of the three launches takes 3 to 12 us for a
+// fraction of a microsecond of traffic: what bounds them is launch and
+// latency, once instead of three times here.  A plane of the slab passes
+// through LDS; the real values of the six components stay in registers.
+// Every pass of data through LDS alternates between two tiles (one barrier
+// each).  Threads hold E values; along z, thread (g, b) holds column b with b
+// fastest; along x, thread (q, g) holds row pair q with g fastest.
+template <typename T, int N>
+struct Slab {
+    // Whole steps, three launches a stage -> one: 16^3 64 -> 53 us, 32^3 71 ->
+    // 69 us, 64^3 FP32 116 -> 105 us.  Not in FP64 at 64^3 (one workgroup a CU
+    // for a chain twice as long, 127 -> 135 us) nor at 48^3 (four short radix
+    // stages along each axis, 103 -> 111 us FP32, 115 -> 137 us FP64)
+    static constexpr bool ok = N <= 32 || (sizeof(T) == 4 && N == 64);
+    static constexpr int E = N == 16 ? 2 : 4;
+    static constexpr int H = N / 2, G = N / E, NT = G * H;
+    static constexpr int XS = N + 1;       // row pairs of a tile along x
+    static constexpr int TILE = H * XS;    // complex values (the z layout [N][H] is smaller)
+    // components that share the exchanges, as LDS allows
+    static constexpr int NC = 3;
+    static_assert(!ok || 2 * NC * TILE * int(sizeof(C2<T>)) <= 131072, "two tiles of three components");
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__((Slab<T, N>::NT))
+k_slab_cross(C2<T>* __restrict__ data, T* __restrict__ ru, const C2<T>* __restrict__ tw, const int* __restrict__ zl,
+             T npoints, size_t bstride) {
+    using SB = Slab<T, N>;
+    constexpr int E = SB::E, H = SB::H, G = SB::G, NT = SB::NT, XS = SB::XS, TILE = SB::TILE;
+    constexpr int NC = SB::NC;
+    constexpr size_t PS = plane_size(N), YS = row_stride(N);
+    using ZI = RegFft<T, N, H, H, NT, +1>;
+    using ZF = RegFft<T, N, H, H, NT, -1>;
+    using XI = RegFft<T, N, 1, 1, G, +1>;
+    using XF = RegFft<T, N, 1, 1, G, -1>;
+    static_assert(ZI::E == E && XI::E == E, "values per thread");
+    __shared__ C2<T> lds[2][NC][TILE];
+    const int y = blockIdx.x, tid = threadIdx.x;
+    data += blockIdx.y * bstride + size_t(y) * YS;
+    if (ru) ru += blockIdx.y * 2 * bstride + size_t(y) * 2 * YS;
+    const T inp = T(1) / npoints;
+    const int b = tid % H, gz = tid / H;   // along z
+    const int gx = tid % G, q = tid / G;   // along x
+    const int lim = zl[b];
+    int cur = 0;
+    // exchange between stage s and s + 1 of the FFTs of NC components: element
+    // addresses by the stage's output and input rows
+    auto exchange = [&](C2<T> (&v)[NC][E], auto&& out_at, auto&& in_at) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) lds[cur][c][out_at(e)] = v[c][e];
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) v[c][e] = lds[cur][c][in_at(e)];
+        cur ^= 1;
+    };
+    auto fft_z = [&](C2<T> (&v)[NC][E], auto f) {
+        using F = decltype(f);
+        sfor<0, F::S>([&](auto s) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) F::template compute_stage<s>(v[c], tw, gz);
+            if constexpr (s + 1 < F::S)
+                exchange(v, [&](int e) { return F::out_row_s(s, gz, e) * H + b; },
+                         [&](int e) { return F::in_row_s(s + 1, gz, e) * H + b; });
+        });
+    };
+    auto fft_x = [&](C2<T> (&v)[NC][E], auto f) {
+        using F = decltype(f);
+        sfor<0, F::S>([&](auto s) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) F::template compute_stage<s>(v[c], tw, gx);
+            if constexpr (s + 1 < F::S)
+                exchange(v, [&](int e) { return q * XS + F::out_row_s(s, gx, e); },
+                         [&](int e) { return q * XS + F::in_row_s(s + 1, gx, e); });
+        });
+    };
+    C2<T> val[6][E];
+    sfor<0, 6 / NC>([&](auto gi) {
+        constexpr int c0 = gi * NC;
+        C2<T> v[NC][E];
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const int n = ZI::in_row(gz, e);
+                v[c][e] = in_band<N>(n, lim) ? data[(c0 + c) * PS + size_t(n) * H + b] : mk<T>(T(0), T(0));
+            }
+        fft_z(v, ZI{});
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) lds[cur][c][ZI::out_row(gz, e) * H + b] = v[c][e];
+        __syncthreads();
+        // rows 2q and 2q + 1 packed, as rows_unpack_inverse
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const int k = XI::in_row(gx, e), kk = k < H ? k : N - k;
+                const C2<T> A = lds[cur][c][2 * q * H + (k == H ? 0 : kk)];
+                const C2<T> Bv = lds[cur][c][(2 * q + 1) * H + (k == H ? 0 : kk)];
+                C2<T> z = k < H ? mk<T>(A.x - Bv.y, A.y + Bv.x) : mk<T>(A.x + Bv.y, Bv.x - A.y);
+                if (k == 0) z = mk<T>(A.x, Bv.x);
+                if (k == H) z = mk<T>(T(0), T(0));
+                v[c][e] = z;
+            }
+        cur ^= 1;
+        fft_x(v, XI{});
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) val[c0 + c][e] = v[c][e];
+    });
+    if (ru) {
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                T* r = ru + c * 2 * PS + 2 * q * N + XI::out_row(gx, e);
+                r[0] = val[c][e].x;
+                r[N] = val[c][e].y;
+            }
+    }
+    // (u x omega) / N^3 on rows gx + G out_m(e), reordered to the forward
+    // FFT's input rows
+    C2<T> f[3][E];
+    sfor<0, E>([&](auto e) {
+        sfor<0, E>([&](auto i) {
+            if constexpr (XI::out_m(i) == XF::in_m(e)) {
+#pragma unroll
+                for (int c = 0; c < 3; c++) {
+                    const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+                    const C2<T> u1 = val[c1][i], u2 = val[c2][i], w1 = val[3 + c1][i], w2 = val[3 + c2][i];
+                    f[c][e] = mk<T>((u1.x * w2.x - u2.x * w1.x) * inp, (u1.y * w2.y - u2.y * w1.y) * inp);
+                }
+            }
+        });
+    });
+    fft_x(f, XF{});
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int e = 0; e < E; e++) lds[cur][c][q * XS + XF::out_row(gx, e)] = f[c][e];
+    __syncthreads();
+    // the rows' spectra, as rows_pack_forward: even z from A, odd from B
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int z = ZF::in_row(gz, e);
+            const C2<T>* row = &lds[cur][c][(z / 2) * XS];
+            const C2<T> Z = row[b], M = row[(N - b) % N];
+            f[c][e] = z % 2 == 0 ? mk<T>(T(0.5) * (Z.x + M.x), T(0.5) * (Z.y - M.y))
+                                 : mk<T>(T(0.5) * (Z.y + M.y), T(-0.5) * (Z.x - M.x));
+        }
+    cur ^= 1;
+    fft_z(f, ZF{});
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            const int n = ZF::out_row(gz, e);
+            if (in_band<N>(n, lim)) data[c * PS + size_t(n) * H + b] = f[c][e];
+        }
 }
 
 // c2r x pass of NC planes into real planes out ([y][z][x] each), components
