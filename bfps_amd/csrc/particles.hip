@@ -959,12 +959,23 @@ struct ColCfg {
     static constexpr int RZ = 2;         // 16-lane row phases per tracer
     static constexpr int LPT = 16 * RZ;  // lanes per tracer
     static constexpr int NI = W / RZ;    // z rows per lane: phase rz takes rows rz NI .. rz NI + NI - 1
-    static constexpr int KX = 32, KZ = 16;
+    // FP64 planes of wider stencils fit as narrower columns: 16 x 16 cells for
+    // n = 4, 5, 16 x 8 for n = 6.  Their halo is a larger part of a slot (n = 6:
+    // 29 x 21 values for 16 x 8 cells), yet no form is faster; velocity loops
+    // with their sorts in us, columns / bricks / gather: 64^3 2 10^4 n4 39 / 44
+    // / 53; 128^3 10^5 n6 250 / 337 / 458; 256^3 2^20 n4 1324 / 2055 / 2573, n6
+    // 2097 / 2883 / 4915; 512^3 2^22 n4 6043 / 11897 / 11374, n6 11014 / 15771 /
+    // 21794
+    static constexpr bool NARROW = sizeof(T) == 8 && NB >= 4;
+    static constexpr int KX = NARROW ? 16 : 32, KZ = NARROW && NB >= 6 ? 8 : 16;
     static constexpr int WX = KX + W - 1, WZ = KZ + W - 1;
     static constexpr int XA = int(16 / sizeof(T));
     static constexpr int XS = (XA - NB % XA) % XA;
     static constexpr int WXT = (WX + XS + XA - 1) / XA * XA;
+    // (the 16 FP64 values of a row phase fill a read cycle by themselves: no
+    // stride between the phases to choose, and no room for padding)
     static constexpr int zs_of(int v) {
+        if (NARROW) return v;
         for (int s = v; s < v + 64 * XA; s += XA)
             if ((NI * s * DW) % 32 == 16) return s;
         return v;
