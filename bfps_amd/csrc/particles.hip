@@ -1634,14 +1634,21 @@ int loop_form(bfpsh_ctx* ctx, int form, const void* u, double dt, int order) {
 // timed on a copy of the tracer state with dt = 0, when it beats the first
 // applicable one by more than 10 % (plan rigor MEASURE or PATIENT, as the
 // pass autotuner), or the first applicable of column walk, bricks, global
-// gather (ESTIMATE).  The trials interpolate ctx->ru, or the field f of nc
+// gather (ESTIMATE).  When a sample of nine planes comes first, the trials are
+// that sample, into its own output: the walks and bricks stage planes whole,
+// the gather reads lines per tracer and plane, so three planes and a move do
+// not tell which is faster for nine (256^3 FP32, 10^5 tracers, n = 4: the loop
+// is fastest by the gather, the gradient sample by columns, 0.63 ms against
+// 0.87 by bricks and 1.37 by the gather).  One form serves the loop and all
+// samples of a tracer set, so that results do not mix forms.
+// The loop's trials interpolate ctx->ru, or the field f of nc
 // planes about to be sampled when ctx->ru is not allocated yet; with
 // neither (a 1-plane sample first) this call takes the first applicable
 // form and the choice waits for a later call.  The forms sum in different
 // orders: results agree to rounding, not bit for bit.  BFPSH_TRACER_VERBOSE
 // set in the environment prints the trials to stderr.
 template <typename T, int NB>
-int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
+int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, double* d_out, int* form) {
     static const char* const names[4] = {"auto", "bricks", "global gather", "column walk"};
     if (ctx->tracer_kernel != FORM_AUTO && form_ok<T, NB>(ctx, ctx->tracer_kernel)) {
         *form = ctx->tracer_kernel;
@@ -1655,7 +1662,8 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
     for (int c : {int(FORM_COLUMN), int(FORM_BRICK), int(FORM_GATHER)})
         if (form_ok<T, NB>(ctx, c)) cand[ncand++] = c;
     int best = cand[0];
-    const void* u = ctx->ru ? ctx->ru : (nc >= 3 ? f : nullptr);
+    const bool nine = nc == 9;
+    const void* u = ctx->ru && !nine ? ctx->ru : (nc >= 3 ? f : nullptr);
     if (ncand > 1 && ctx->plan_rigor != BFPSH_ESTIMATE && ctx->tracer_kernel == FORM_AUTO && !u) {
         *form = best;
         return BFPSH_OK;
@@ -1669,23 +1677,30 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
         const size_t rhs_bytes = size_t(ctx->nsteps) * pos_bytes;
         double *spos = nullptr, *srhs = nullptr;
         hipEvent_t a = nullptr, b = nullptr;
-        HIPCHK(hipMalloc((void**)&spos, pos_bytes));
-        if (hipMalloc((void**)&srhs, rhs_bytes) != hipSuccess) {
-            (void)hipFree(spos);
-            return fail(ctx, BFPSH_EHIP, "tracer kernel choice: device memory for the trial state");
+        if (!nine) {
+            HIPCHK(hipMalloc((void**)&spos, pos_bytes));
+            if (hipMalloc((void**)&srhs, rhs_bytes) != hipSuccess) {
+                (void)hipFree(spos);
+                return fail(ctx, BFPSH_EHIP, "tracer kernel choice: device memory for the trial state");
+            }
+            HIPCHK(hipMemsetAsync(srhs, 0, rhs_bytes, ctx->stream));
         }
-        HIPCHK(hipMemsetAsync(srhs, 0, rhs_bytes, ctx->stream));
         HIPCHK(hipEventCreate(&a));
         HIPCHK(hipEventCreate(&b));
         double* const pos = ctx->d_pos;
         double* const rhs = ctx->d_rhs;
         const bool prof = ctx->prof, add_head = ctx->add_head;
         ctx->prof = false;  // the trials stay out of the kernel profile
-        ctx->d_pos = spos;
-        ctx->d_rhs = srhs;
+        if (!nine) {
+            ctx->d_pos = spos;
+            ctx->d_rhs = srhs;
+        }
         ctx->add_head = false;
+        auto trial = [&](int c) -> int {
+            return nine ? sample_form<T, NB>(ctx, c, u, 9, d_out) : loop_form<T, NB>(ctx, c, u, 0.0, ctx->nsteps);
+        };
         auto fresh = [&]() -> int {
-            if (hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+            if (!nine && hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
                 return BFPSH_EHIP;
             ctx->sort_age = 1 << 30;  // bricks and columns sort, as in a step
             return BFPSH_OK;
@@ -1694,21 +1709,22 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
         int r = BFPSH_OK;
         for (int i = 0; i < ncand && r == BFPSH_OK; i++) {
             r = fresh();
-            if (r == BFPSH_OK) r = loop_form<T, NB>(ctx, cand[i], u, 0.0, ctx->nsteps);  // warm-up
+            if (r == BFPSH_OK) r = trial(cand[i]);  // warm-up
             if (r == BFPSH_OK) r = fresh();
             // (the gather renews its permutation every sort_every steps: it
             // is timed on the one of its warm-up)
             if (cand[i] == FORM_GATHER && ctx->sort_every > 1) ctx->sort_age = 0;
             if (r == BFPSH_OK && hipEventRecord(a, ctx->stream) != hipSuccess) r = BFPSH_EHIP;
-            if (r == BFPSH_OK) r = loop_form<T, NB>(ctx, cand[i], u, 0.0, ctx->nsteps);
+            if (r == BFPSH_OK) r = trial(cand[i]);
             float ms = 0.f;
             if (r == BFPSH_OK && (hipEventRecord(b, ctx->stream) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
                                   hipEventElapsedTime(&ms, a, b) != hipSuccess))
                 r = BFPSH_EHIP;
             if (i == 0) tfirst = ms;
             if (r == BFPSH_OK && std::getenv("BFPSH_TRACER_VERBOSE"))
-                std::fprintf(stderr, "bfpsh: tracer form trial (n = %d, %s tracers, %lld of them): %s %.3f ms\n",
-                             NB, sizeof(T) == 8 ? "FP64" : "FP32", (long long)ctx->np, names[cand[i]], ms);
+                std::fprintf(stderr, "bfpsh: tracer form trial (n = %d, %s tracers, %lld of them%s): %s %.3f ms\n",
+                             NB, sizeof(T) == 8 ? "FP64" : "FP32", (long long)ctx->np,
+                             nine ? ", 9-plane sample" : "", names[cand[i]], ms);
             if (r == BFPSH_OK && ms < tbest) {
                 tbest = ms;
                 best = cand[i];
@@ -1740,7 +1756,7 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, int* form) {
 template <typename T, int NB>
 int loop_nb(bfpsh_ctx* ctx, double dt, int order) {
     int form = FORM_GATHER;
-    int r = tracer_form<T, NB>(ctx, ctx->ru, 3, &form);
+    int r = tracer_form<T, NB>(ctx, ctx->ru, 3, nullptr, &form);
     if (r) return r;
     return loop_form<T, NB>(ctx, form, ctx->ru, dt, order);
 }
@@ -1748,7 +1764,7 @@ int loop_nb(bfpsh_ctx* ctx, double dt, int order) {
 template <typename T, int NB>
 int sample_nb(bfpsh_ctx* ctx, const void* f, int nc, double* d_out) {
     int form = FORM_GATHER;
-    int r = tracer_form<T, NB>(ctx, f, nc, &form);
+    int r = tracer_form<T, NB>(ctx, f, nc, d_out, &form);
     if (r) return r;
     return sample_form<T, NB>(ctx, form, f, nc, d_out);
 }
