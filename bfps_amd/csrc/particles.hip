@@ -1696,8 +1696,8 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, double* d_out, int* form)
             ctx->d_rhs = srhs;
         }
         ctx->add_head = false;
-        auto trial = [&](int c) -> int {
-            return nine ? sample_form<T, NB>(ctx, c, u, 9, d_out) : loop_form<T, NB>(ctx, c, u, 0.0, ctx->nsteps);
+        auto trial = [&](int c, int planes) -> int {
+            return nine ? sample_form<T, NB>(ctx, c, u, planes, d_out) : loop_form<T, NB>(ctx, c, u, 0.0, ctx->nsteps);
         };
         auto fresh = [&]() -> int {
             if (!nine && hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
@@ -1708,18 +1708,29 @@ int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, double* d_out, int* form)
         double tbest = 1e300, tfirst = 0.0;
         int r = BFPSH_OK;
         for (int i = 0; i < ncand && r == BFPSH_OK; i++) {
-            r = fresh();
-            if (r == BFPSH_OK) r = trial(cand[i]);  // warm-up
-            if (r == BFPSH_OK) r = fresh();
-            // (the gather renews its permutation every sort_every steps: it
-            // is timed on the one of its warm-up)
-            if (cand[i] == FORM_GATHER && ctx->sort_every > 1) ctx->sort_age = 0;
-            if (r == BFPSH_OK && hipEventRecord(a, ctx->stream) != hipSuccess) r = BFPSH_EHIP;
-            if (r == BFPSH_OK) r = trial(cand[i]);
             float ms = 0.f;
-            if (r == BFPSH_OK && (hipEventRecord(b, ctx->stream) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-                                  hipEventElapsedTime(&ms, a, b) != hipSuccess))
-                r = BFPSH_EHIP;
+            auto timed = [&](int planes) -> int {
+                if (hipEventRecord(a, ctx->stream) != hipSuccess) return BFPSH_EHIP;
+                const int q = trial(cand[i], planes);
+                if (q) return q;
+                return hipEventRecord(b, ctx->stream) == hipSuccess && hipEventSynchronize(b) == hipSuccess &&
+                               hipEventElapsedTime(&ms, a, b) == hipSuccess
+                           ? BFPSH_OK
+                           : BFPSH_EHIP;
+            };
+            r = fresh();
+            // warm-up: the first form's may load the code (14 ms), three planes
+            // do; a later form's nine planes that take above 1 ms and longer
+            // than a form timed before are not repeated (2^19 tracers, n = 6,
+            // 256^3: first gradient sample 30.7 -> 19.4 ms)
+            if (r == BFPSH_OK) r = timed(nine && i > 0 ? 9 : 3);
+            if (r == BFPSH_OK && !(nine && i > 0 && ms > 1.f && ms > tbest)) {
+                r = fresh();
+                // (the gather renews its permutation every sort_every steps:
+                // it is timed on the one of its warm-up)
+                if (cand[i] == FORM_GATHER && ctx->sort_every > 1) ctx->sort_age = 0;
+                if (r == BFPSH_OK) r = timed(nine ? 9 : 3);
+            }
             if (i == 0) tfirst = ms;
             if (r == BFPSH_OK && std::getenv("BFPSH_TRACER_VERBOSE"))
                 std::fprintf(stderr, "bfpsh: tracer form trial (n = %d, %s tracers, %lld of them%s): %s %.3f ms\n",

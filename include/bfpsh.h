@@ -75,7 +75,8 @@ int bfpsh_create(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky
  * the first tracer loop or sample of a tracer set also times the velocity
  * loop of each applicable tracer kernel form (column walk, bricks, global
  * gather) on a device copy of the tracer state, which it allocates for the
- * time it runs, and keeps the fastest when it is more than 10 % faster
+ * time it runs (or the 9-plane sample itself, where that comes first), and
+ * keeps the fastest when it is more than 10 % faster
  * than the first applicable one (BFPSH_TRACER_KERNEL=column|brick|gather
  * in the environment forces a form, BFPSH_TRACER_VERBOSE prints the
  * trials). */
