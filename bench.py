@@ -48,31 +48,40 @@ WORKLOADS = {
 }
 
 
-def step_bytes(n, es, with_tracer_u):
-    """Algorithmic HBM bytes of one fused vorticity step: 141 field volumes
-    (N^3 elements of size es) + 3 for the real velocity handed to the
-    tracers."""
-    return (141 + (3 if with_tracer_u else 0)) * n ** 3 * es
-
-
-# algorithmic bytes per launch of each kernel, in field volumes N^3 * es
-# ("inv_z_bs" is reported as one kernel: the kx tile holding kx = 0 runs as a
-# separate launch "inv_z_bs_t0" with the symmetrize mirror, merged below)
+# algorithmic bytes per launch of each kernel, in field volumes N^3 * es of
+# whole planes: under the smooth filter the state fills the sphere |k| <= N/2,
+# SPHERE of a spectral plane, and the passes move only the columns (kz, kx)
+# inside it, BAND of a plane
+BAND, SPHERE = 3.141592653589793 / 4, 3.141592653589793 / 6
 KERNEL_VOLUMES = {
-    "inv_z_bs": 9,         # read omega (3 planes), write u, omega after the z pass (6)
-    "inv_y": 12,           # 6 planes read + written
-    "rows_cross": 9,       # read 6, write 3 (+3 real velocity in stage 1)
-    "fwd_z": 6,            # 3 planes read + written
-    "fwd_y_update1": 9,    # read N (3), v0 (3), write v1 (3)
-    "fwd_y_update2": 12,   # read N, v0, v1, write v2
-    "fwd_y_update3": 12,   # read N, v0, v2, write v0
+    "bs_inv_y": 3 * SPHERE + 6 * BAND,    # read omega, write u, omega after the y pass
+    "inv_y": 12,                          # 6 planes read + written
+    "inv_z": 6 * BAND + 6,                # 6 planes
+    "rows_cross": 9,                      # read 6, write 3 (+3 real velocity in stage 1)
+    "fwd_z": 3 + 3 * BAND,                # 3 planes
+    "y_update1": 9 * BAND + 6 * SPHERE,   # read N, v0, write v1 and u, omega of stage 2
+    "y_update2": 9 * BAND + 9 * SPHERE,   # read N, v0, v1, write v2 and u, omega of stage 3
+    "y_update3": 3 * BAND + 9 * SPHERE,   # read N, v0, v2, write v0
 }
+
+
+def step_bytes(n, es, with_tracer_u):
+    """Algorithmic HBM bytes of one fused vorticity step: the first pass,
+    three times inverse z, x with the cross product and forward z, and the
+    three updates (110.5 field volumes; 135 of whole planes), + 3 for the real
+    velocity handed to the tracers."""
+    k = KERNEL_VOLUMES
+    vols = (k["bs_inv_y"] + 3 * (k["inv_z"] + k["rows_cross"] + k["fwd_z"]) + k["y_update1"] + k["y_update2"] +
+            k["y_update3"])
+    return int((vols + (3 if with_tracer_u else 0)) * n ** 3 * es)
+
+
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_%d_fp32.txt")
 
 
 def merge_profile(prof):
-    """Fold the kx-tile-0 launch of the Biot-Savart pass into "inv_z_bs";
-    the tracer velocity loop is "interp_ab" whichever kernel form ran (the
+    """Fold the kx-tile-0 launch "inv_z_bs_t0" of a Biot-Savart z pass, where
+    a profile holds one, into "inv_z_bs"; the tracer velocity loop is "interp_ab" whichever kernel form ran (the
     column walk and the global gather are profiled as "interp_ab_col" and
     "interp_ab_gather")."""
     out = dict(prof)
@@ -233,7 +242,7 @@ def roofline(prof, n, es, np_, nb, traffic_ok, steps):
         xa = 16 // es
         xs = (xa - nb % xa) % xa
         if form == "column walk":
-            kx, kz = 32, 16
+            kx, kz = (32, 16) if es == 4 or nb < 4 else (16, 16 if nb < 6 else 8)
             wxt = (kx + w - 1 + xs + xa - 1) // xa * xa
             windows = 3 * (n // kx) * (n // kz) * (n + w - 1) * wxt * (kz + w - 1)
         else:
