@@ -193,7 +193,8 @@ template <int MODE> struct BsOut { static constexpr int NF = MODE == 0 ? 6 : (MO
 // upper half (field.cpp:900-978).  The c2r pass takes the real part of the
 // kx = 0 sum, to which a mode and its conjugated mirror add the same, so the
 // lower half may be left out and the upper half doubled: this factor of a
-// kx = 0 mode, with no mirror to read.
+// kx = 0 mode, with no mirror to read.  (A z derivative at kz = N/2, whose
+// mirror has the same kz, is no such pair: see MODE 2 below.)
 template <typename T, int N> BFPSH_DEV T plane0_factor(int ky, int kz) {
     if (ky > N / 2 || (ky == 0 && kz > N / 2)) return T(0);
     if (ky == N / 2 || (ky == 0 && (kz == 0 || kz == N / 2))) return T(1);  // its own mirror, or none
@@ -268,7 +269,11 @@ BFPSH_DEV void bs_inverse_y(C2<T> (&wr)[3][E], C2<T>* lds, int cur, const C2<T>*
             if (MODE == 2) {
                 const int j = f / 3;
                 const double kj = j == 0 ? kx : (j == 1 ? kyv : kzv);
-                v[e] = k2 < g.kM2 ? mk<T>(T(-kj * u.y), T(kj * u.x)) : mk<T>(T(0), T(0));
+                // i k_z of a kx = 0 mode at kz = N/2 and of its mirror, both
+                // at +N/2: their sum has no real part, where doubling one
+                // counts the part that the mirror cancels
+                const bool cancels = kxi == 0 && j == 2 && kz == N / 2 && n > 0 && n < N / 2;
+                v[e] = k2 < g.kM2 && !cancels ? mk<T>(T(-kj * u.y), T(kj * u.x)) : mk<T>(T(0), T(0));
             } else {
                 v[e] = u;
             }

@@ -65,6 +65,33 @@ def test_step(oracle, n, dealias, projected, dk, nu):
     assert e < TOL
 
 
+@pytest.mark.parametrize("n, dealias, dk", [
+    (32, "SMOOTH", (1.0, 1.0, 1.0)),
+    # ky = n/2 and kz = n/2 inside the sphere
+    (64, "SMOOTH", (1.0, 0.5, 0.75)),
+    (32, "TWO_THIRDS", (1.25, 1.0, 0.5)),
+])
+def test_gradient(oracle, n, dealias, dk):
+    """Velocity and its gradient in real space, component by component."""
+    import bfps_amd as B
+    print("case: band gradient n=%d %s dk=%s" % (n, dealias, dk), flush=True)
+    fs = B.vorticity_equation("t", n, dkx=dk[0], dky=dk[1], dkz=dk[2], precision="double", dealias=dealias)
+    o = oracle.Solver(n, precision="double", dealias=dealias, dk=dk)
+    w0 = spectrum(n, n + 1)
+    fs.io_checkpoint(read=True, data=w0)
+    o.set_cfield("vorticity", w0)
+    o.io_projection()
+    fs.velocity_rspace()
+    o.velocity_rspace()
+    assert rel(fs.get_rfield(B.capi.RVELOCITY), o.get_rfield("rvelocity")) < TOL
+    fs.gradient_rspace()
+    o.gradient_rspace()
+    got, want = fs.get_rfield(B.capi.RGRADIENT), o.get_rfield("gradient")
+    errors = [rel(got[..., c], want[..., c]) for c in range(9)]
+    print("  rel", errors, flush=True)
+    assert max(errors) < TOL
+
+
 def test_put_switches_the_table(oracle):
     """An unprojected put, then a projection, then steps: each form in turn,
     and the same in a box of an ensemble beside a projected one."""
