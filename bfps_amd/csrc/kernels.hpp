@@ -1085,6 +1085,36 @@ k_rows_r2c(const T* data, C2<T>* out, const C2<T>* __restrict__ tw) {
     }
 }
 
+// ------------------------------------------------------------ integrating factor
+// exp(x + y) as `one` + a b + (a lb + la b) from a part a, la of x and b, lb
+// of y, which depend on fewer indexes than their sum.  While the factors stay
+// above exp(-1/2) (`slow`, uniform; one = 1), a = exp(x) - 1 and la = 1: 1 +
+// (a + b + a b), whose error is that of its last rounding, like an
+// exponential's own.  Beyond (one = 0), that sum would cancel, and a product
+// of two rounded exponentials has 1.3 times an exponential's error: there
+// exp(x) = a + la, a its rounded value and la the rest, from x = m ln 2 + r,
+// |r| <= ln 2 / 2 (argument reduction of Cody and Waite) and exp(r) - 1.
+// FP64 decay at 64^3 over 64 steps, mean error of a mode at nu dt kM^2 = 1.4 /
+// 3: 7.8e-15 / 1.00e-14; by products 1.02e-14 / 1.29e-14; with one rounded
+// exponential a factor 8.3e-15 / 9.7e-15.
+BFPSH_DEV double if_part(double x, bool slow, float& rest) {
+    double q = 0.0;
+    if (!slow) {
+        q = rint(fmin(fmax(x * 0x1.71547652b82fep+0, -8000.0), 8000.0));  // x / ln 2
+        // (ln 2 and what its rounding leaves)
+        x = fma(-q, 0x1.abc9e3b39803fp-56, fma(-q, 0x1.62e42fefa39efp-1, x));
+    }
+    const double e = expm1(x);
+    rest = 1.0f;
+    if (slow) return e;
+    const double h = 1.0 + e;
+    rest = float(ldexp(e - (h - 1.0), int(q)));
+    return ldexp(h, int(q));
+}
+BFPSH_DEV double if_of(double a, double b, float la, float lb, double one) {
+    return one + fma(a, b, fma(a, double(lb), double(la) * b));
+}
+
 // ------------------------------------------------------------ last forward pass + update
 // STAGE 1..3 of the integrating-factor SSP-RK3 step
 // (vorticity_equation::step, bfps/cpp/vorticity_equation.cpp:358-439), fused
@@ -1102,10 +1132,7 @@ k_rows_r2c(const T* data, C2<T>* out, const C2<T>* __restrict__ tw) {
 // as zeros); stage 3 keeps v0 there, projected, when `full` says that it may
 // hold something.  The integrating factor exp(-nu k^2 dt c) is combined from
 // one value per ky, in an LDS table, and one per thread for its (kx, kz),
-// instead of one exponential per mode (two in stage 2): from
-// e = exp - 1 as 1 + (a + b + a b), whose error is that of its last rounding
-// like the exponential's own, while the factors stay above exp(-1/2); the
-// product of exponentials where viscosity damps the last modes faster.
+// instead of one exponential per mode (two in stage 2): see if_of.
 template <typename T, int N, int STAGE, bool BATCH, int E_ = Cfg<T, N>::E_Y3, int B_ = Cfg<T, N>::B_Y3>
 __global__ void __launch_bounds__(((N / E_) * B_))
 k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* __restrict__ tw,
@@ -1128,6 +1155,7 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     constexpr int NBUF = fused_bufs<T, N>(B);
     __shared__ C2<T> lds[NBUF * N * B];
     __shared__ double ify[STAGE == 2 ? 2 : 1][N];
+    __shared__ float ifr[STAGE == 2 ? 2 : 1][N];
     const int tid = threadIdx.x;
     const int b = tid % B, grp = tid / B;
     // tiles narrower than a 128-byte line (1024^3): neighbouring tiles, the
@@ -1151,15 +1179,15 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     const double kx = kxi * g.dkx, kzv = kwave(kz, N, g.dkz);
     const double dt = sp.dt, nud = sp.nu * dt * (STAGE == 1 ? 1.0 : 0.5);
     const bool slow = fabs(nud) * g.kM2 < 0.5;  // uniform
-    auto if_part = [&](double x) { return slow ? expm1(x) : exp(x); };
-    auto if_of = [&](double p, double q) { return slow ? 1.0 + fma(p, q, p + q) : p * q; };
     for (int i = tid; i < N; i += NT) {
         const double k = kwave(i, N, g.dky);
-        ify[0][i] = if_part(-nud * k * k);
-        if constexpr (STAGE == 2) ify[1][i] = if_part(nud * k * k);
+        ify[0][i] = if_part(-nud * k * k, slow, ifr[0][i]);
+        if constexpr (STAGE == 2) ify[1][i] = if_part(nud * k * k, slow, ifr[1][i]);
     }
-    const double ifxz = if_part(-nud * (kx * kx + kzv * kzv));
-    const double ifxz1 = STAGE == 2 ? if_part(nud * (kx * kx + kzv * kzv)) : 0.0;
+    const double one = slow ? 1.0 : 0.0;
+    float rxz, rxz1 = 0.f;
+    const double ifxz = if_part(-nud * (kx * kx + kzv * kzv), slow, rxz);
+    const double ifxz1 = STAGE == 2 ? if_part(nud * (kx * kx + kzv * kzv), slow, rxz1) : 0.0;
     __syncthreads();
     // one component after the other; an opaque group index and table offset
     // per component, so that twiddles and LDS addresses are not held across,
@@ -1247,13 +1275,13 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
             const double ik2 = k2 > 0 ? 1.0 / k2 : 0.0;  // one division, then products
             if (k2 > 0) divfree<T>(cu, kx, kyv, kzv, ik2);
             else cu[0] = cu[1] = cu[2] = mk<T>(T(0), T(0));
-            const double f0 = if_of(ifxz, ify[0][ky]);
+            const double f0 = if_of(ifxz, ify[0][ky], rxz, ifr[0][ky], one);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 if constexpr (STAGE == 1) {
                     nv[c] = mk<T>(T((w0[c].x + dt * cu[c].x) * f0), T((w0[c].y + dt * cu[c].y) * f0));
                 } else if constexpr (STAGE == 2) {
-                    const double f1 = if_of(ifxz1, ify[STAGE - 1][ky]);
+                    const double f1 = if_of(ifxz1, ify[STAGE - 1][ky], rxz1, ifr[STAGE - 1][ky], one);
                     nv[c] = mk<T>(T((3 * w0[c].x * f0 + (w1[c].x + dt * cu[c].x) * f1) * 0.25),
                                   T((3 * w0[c].y * f0 + (w1[c].y + dt * cu[c].y) * f1) * 0.25));
                 } else {
