@@ -207,7 +207,7 @@ struct Impl {
                 // grow with each transform, and zeros move and compute at
                 // other speeds (512^3 FP32 forward z pass on zeros: the
                 // slowest of four candidates, 0.675 against 0.58 ms, won)
-                k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>((T*)ctx->work, 6 * ctx->ps);
+                k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>((CT*)ctx->work, 6 * ctx->ps);
                 run();  // warm-up
                 (void)hipEventRecord(a, ctx->stream);
                 for (int r = 0; r < reps; r++) run();

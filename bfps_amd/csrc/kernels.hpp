@@ -1388,10 +1388,12 @@ __global__ void __launch_bounds__(256) k_band_amplitude(const C2<T>* __restrict_
 }
 
 // ------------------------------------------------------------ small spectral kernels
-// data of the autotuner's trials: values in [-1, 1) without a pattern
-template <typename T> __global__ void __launch_bounds__(256) k_fill_pattern(T* d, size_t count) {
+// data of the autotuner's trials: `count` complex values in the unit square
+// without a pattern
+template <typename T> __global__ void __launch_bounds__(256) k_fill_pattern(C2<T>* d, size_t count) {
+    auto value = [](size_t i) { return T(int32_t(uint32_t(i) * 2654435761u)) * T(1.0 / 2147483648.0); };
     for (size_t i = size_t(blockIdx.x) * 256 + threadIdx.x; i < count; i += size_t(gridDim.x) * 256)
-        d[i] = T(int32_t(uint32_t(i) * 2654435761u)) * T(1.0 / 2147483648.0);
+        d[i] = mk<T>(value(2 * i), value(2 * i + 1));
 }
 
 // field::symmetrize on the kx = 0 plane (bfps/cpp/field.cpp:900-978):
