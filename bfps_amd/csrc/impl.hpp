@@ -152,6 +152,7 @@ struct Impl {
             int r = ensure_work(ctx, 6);
             if (r) return r;
         }
+        CT* scratch = nullptr;
         hipEvent_t a = nullptr, b = nullptr;
         int rc = BFPSH_OK;
         for (int kind = 0; kind < BFPSH_PASS_KINDS && rc == BFPSH_OK; kind++) {
@@ -172,6 +173,14 @@ struct Impl {
                     break;
                 }
             }
+            // the fused passes read a vorticity and write a stage: three planes
+            // of their own, without which (no memory) the built-in shape stays
+            const bool fused = kind == BFPSH_PASS_BS || kind == BFPSH_PASS_Y3;
+            if (fused && !scratch && hipMalloc((void**)&scratch, 3 * ctx->ps * sizeof(CT)) != hipSuccess) {
+                (void)hipGetLastError();
+                scratch = nullptr;
+                continue;
+            }
             // two rounds over the shapes, the better time of each: the first
             // trials of a round run while the clocks still rise
             const int rounds = 2, reps = rigor >= BFPSH_PATIENT ? 5 : 2;
@@ -183,19 +192,20 @@ struct Impl {
                 // one launch of shape v: a plain pass over the planes of a step
                 // (one plane would stay in the last-level cache, where other
                 // shapes win), the z passes within the band as the step runs
-                // them; the first pass from cvorticity into the work planes; the
-                // last pass of stage 1 from the work planes into v1 (which
-                // every step writes before it reads it) and back into them
+                // them; the first pass from the scratch planes into the work
+                // planes; the last pass of stage 1 from the work planes and the
+                // scratch planes back into both, with dt = 0, which keeps the
+                // values as they are
                 auto run = [&]() {
                     if (kind == BFPSH_PASS_BS) {
-                        bs_fn(v)(ctx->stream, (const CT*)ctx->v0, (CT*)ctx->work, tw, band(ctx), ctx->outside,
-                                 geom(ctx));
+                        bs_fn(v)(ctx->stream, scratch, (CT*)ctx->work, tw, band(ctx), ctx->outside, geom(ctx));
                     } else if (kind == BFPSH_PASS_Y3) {
                         StepParams sp = ctx->sp;
                         sp.forcing = BFPSH_FORCING_NONE;
                         sp.famp_dev = nullptr;
-                        y3_fn(1, v)(ctx->stream, (CT*)ctx->work, (const CT*)ctx->v0, (const CT*)ctx->v1,
-                                    (CT*)ctx->v1, tw, band(ctx), ctx->outside, geom(ctx), sp);
+                        sp.dt = 0.0;
+                        y3_fn(1, v)(ctx->stream, (CT*)ctx->work, scratch, scratch, scratch, tw, band(ctx), ctx->outside,
+                                    geom(ctx), sp);
                     } else {
                         const bool z = kind == BFPSH_PASS_Z_INV || kind == BFPSH_PASS_Z_FWD;
                         const int planes = kind == BFPSH_PASS_Z_INV ? 6 : 3;
@@ -208,6 +218,7 @@ struct Impl {
                 // other speeds (512^3 FP32 forward z pass on zeros: the
                 // slowest of four candidates, 0.675 against 0.58 ms, won)
                 k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>((CT*)ctx->work, 6 * ctx->ps);
+                if (fused) k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>(scratch, 3 * ctx->ps);
                 run();  // warm-up
                 (void)hipEventRecord(a, ctx->stream);
                 for (int r = 0; r < reps; r++) run();
@@ -237,6 +248,10 @@ struct Impl {
         }
         if (a) (void)hipEventDestroy(a);
         if (b) (void)hipEventDestroy(b);
+        if (scratch) {
+            (void)hipStreamSynchronize(ctx->stream);
+            (void)hipFree(scratch);
+        }
         return rc;
     }
 

@@ -276,10 +276,11 @@ int bfpsh_device_bytes(bfpsh_ctx* ctx, size_t* bytes);
 /* Replaces the plan creation with `plan_rigor` in the field constructor
  * (bfps/cpp/field.cpp:105-118): chooses the tile shape of each strided pass
  * kind of this context by `rigor` (BFPSH_ESTIMATE / MEASURE / PATIENT, see
- * above).  As FFTW_MEASURE overwrites the arrays it plans for, measuring
- * overwrites the context's work planes (the spectral velocity of
- * compute_velocity) and the first Runge-Kutta stage, which every step writes
- * before it reads it; the vorticity is left untouched. */
+ * above).  Measuring allocates three planes for the time it runs (boxes of
+ * 512^3 and more; without them the fused passes keep their built-in shapes)
+ * and, as FFTW_MEASURE overwrites the arrays it plans for, overwrites the
+ * context's work planes (the spectral velocity of compute_velocity); the
+ * vorticity and the Runge-Kutta stages are left untouched. */
 int bfpsh_set_plan_rigor(bfpsh_ctx* ctx, int rigor);
 /* The tile shape in use for pass `kind` (BFPSH_PASS_*): e complex values per
  * thread, b columns per tile, persistent = 1 for the form whose workgroups
