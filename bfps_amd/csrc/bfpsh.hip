@@ -191,6 +191,9 @@ int create_ctx(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky, 
         if (zl[x] >= 0) zl[nh] = x;
     }
     ctx->xl = zl[nh];
+    int64_t pencils = 0;
+    for (int x = 0; x <= ctx->xl; x++) pencils += std::min(2 * zl[x] + 1, n);
+    ctx->band_percent = int(100 * pencils / (int64_t(n) * nh));
     // twiddles and tables in one buffer
     const size_t twb = tw.size();
     tw.resize(twb + zl.size() * sizeof(int));
@@ -759,7 +762,11 @@ namespace {
 std::mutex wisdom_mu;
 std::map<std::string, PassWisdom> wisdom;
 std::map<int, std::string> arch_names;  // device -> architecture (gcnArchName up to ':')
-const char* const kPassKindName[BFPSH_PASS_KINDS] = {"z_inv", "y_inv", "z_fwd", "y_fwd", "bs", "y3"};
+// Named after what a search of the kind times: entries of another name (a file
+// of a build whose trials or kernels differed: z_inv, y_inv, z_fwd and y_fwd
+// timed on one plane, bs and y3 along other axes) are kept and never used.
+const char* const kPassKindName[BFPSH_PASS_KINDS] = {"z_inv_band", "y_inv_planes", "z_fwd_band", "y_fwd_planes",
+                                                     "bs_inv_y", "y_update"};
 }  // namespace
 
 std::string pass_wisdom_key(const bfpsh_ctx* ctx, int kind) {
@@ -779,8 +786,14 @@ std::string pass_wisdom_key(const bfpsh_ctx* ctx, int kind) {
         std::lock_guard<std::mutex> lk(wisdom_mu);
         arch_names[ctx->device] = arch;
     }
-    return arch + "/" + (ctx->prec == BFPSH_FP32 ? "f32" : "f64") + "/" + std::to_string(ctx->n) + "/" +
-           kPassKindName[(kind >= 0 && kind < BFPSH_PASS_KINDS) ? kind : 0];
+    if (kind < 0 || kind >= BFPSH_PASS_KINDS) kind = 0;
+    std::string key = arch + "/" + (ctx->prec == BFPSH_FP32 ? "f32" : "f64") + "/" + std::to_string(ctx->n) + "/" +
+                      kPassKindName[kind];
+    // the trials within the band: its share of the pencils, in percent, stands
+    // for the dealiasing rule and the wavenumber units (SMOOTH 78, TWO_THIRDS 34)
+    if (kind != BFPSH_PASS_Y_INV && kind != BFPSH_PASS_Y_FWD)
+        key += std::to_string(ctx->outside ? 100 : ctx->band_percent);
+    return key;
 }
 
 bool pass_wisdom_lookup(const std::string& key, PassWisdom* w) {

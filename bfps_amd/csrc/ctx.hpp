@@ -47,6 +47,7 @@ struct bfpsh_ctx {
     const int* zl = nullptr;       // band table of the sphere, then of the whole half spectrum (n/2 + 1 ints
                                    // each), behind the twiddles
     int xl = 0;                    // largest kx index inside the sphere
+    int band_percent = 100;        // of the (kx, kz) pencils, those that reach the sphere
     int outside = 0;               // 1: v0 may hold modes outside the sphere (put, not projected since)
     double* d_famp = nullptr;      // per-stage band amplitude (fixed energy-injection forcing)
     bool ru_valid = false;
@@ -237,9 +238,10 @@ struct OpsTable {
 };
 
 // Process-wide pass wisdom (bfpsh.hip): the tile shape the autotuner chose
-// for one (GPU architecture, precision, N, pass kind), with its time per
-// plane and the rigor of the search that chose it.  Keys are
-// "arch/f32|f64/N/kind".
+// for one (GPU architecture, precision, N, pass kind, band), with the time of
+// its launch and the rigor of the search that chose it.  Keys are
+// "arch/f32|f64/N/kind", the kind followed by the band's percent of the pencils
+// where the pass keeps within it.
 struct PassWisdom {
     int e = 0, b = 0, pp = 0;
     double ms = 0.0;

@@ -295,6 +295,9 @@ int bfpsh_set_pass_shape(bfpsh_ctx* ctx, int kind, int index);
  * (bfps/cpp/full_code/main_code.hpp:101-104,145-149) and fftw_forget_wisdom:
  * the process-wide pass wisdom as a text file, one line per (architecture,
  * precision, N, pass kind): "<arch>/<f32|f64>/<N>/<kind> <e> <b> <persistent> <ms> <rigor>".
+ * The kinds of the step's passes carry the percent of the pencils inside the
+ * dealiasing sphere.  Entries of kinds that this library does not have (files
+ * of another build) are kept and not used.
  * Importing a missing file is not an error (as the reference's start of a
  * new simulation); lines that do not parse are rejected. */
 int bfpsh_wisdom_import(const char* path);

@@ -309,3 +309,39 @@ def test_plan_rigor_and_wisdom(B, tmp_path):
         fs4 = B.vorticity_equation("t4", 32, precision="single", plan_rigor="FFTW_WHATEVER")
         fs4.close()
     B.wisdom_forget()
+
+
+def test_wisdom_of_other_trials_is_not_used(B, tmp_path):
+    """Entries of kinds whose trials or kernels differ (a file of an earlier
+    build: z_inv, bs, ...) do not choose a shape, and a search under one
+    dealiasing rule does not choose the shapes of the passes within another
+    rule's band, while plain y passes share theirs."""
+    say("case: wisdom of other trials")
+    B.wisdom_forget()
+    probe = B.vorticity_equation("t", 256, precision="single", plan_rigor="FFTW_ESTIMATE")
+    shapes = {k: [] for k in ("z_inv", "y_inv", "z_fwd", "y_fwd")}
+    for k in shapes:
+        for i in range(probe.pass_shapes()[k][3]):
+            probe.set_pass_shape(k, i)
+            e, b, _, _, pp = probe.pass_shapes()[k]
+            shapes[k].append((e, b, pp))
+    probe.close()
+    old = tmp_path / "old.txt"
+    old.write_text("".join("gfx950/f32/256/%s %d %d %d 0.01 2\n" % ((k,) + v[-1]) for k, v in shapes.items()))
+    B.wisdom_import(str(old))
+    fs = B.vorticity_equation("t", 256, precision="single", plan_rigor="FFTW_ESTIMATE")
+    assert all(v[2] == 0 for v in fs.pass_shapes().values())
+    fs.close()
+    B.wisdom_forget()
+
+    def searched():
+        path = str(tmp_path / "w.txt")
+        B.wisdom_export(path)
+        return {l.split()[0] for l in open(path) if not l.startswith("#")}
+
+    B.vorticity_equation("t", 256, precision="single", dealias="TWO_THIRDS", plan_rigor="FFTW_MEASURE").close()
+    first = searched()
+    B.vorticity_equation("t", 256, precision="single", plan_rigor="FFTW_MEASURE").close()
+    both = searched()
+    assert len(first) == 4 and len(both) == 6 and first < both
+    B.wisdom_forget()
