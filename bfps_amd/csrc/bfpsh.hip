@@ -590,7 +590,8 @@ int bfpsh_particles_create(bfpsh_ctx* ctx, int64_t np, int n, int m, int nsteps,
                              : !std::strcmp(tk, "gather") ? 2
                              : !std::strcmp(tk, "column") ? 3
                                                           : 0;
-        ctx->tracer_form = 0;
+        ctx->tracer_form = ctx->nine_form = 0;
+        ctx->nine_sampled = ctx->looped = false;
     }
     ctx->nsteps = nsteps;
     ctx->step_idx = step_idx;

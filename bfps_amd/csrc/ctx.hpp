@@ -33,6 +33,9 @@ struct bfpsh_ctx {
     bool force_coop = false;       // tracers: global-gather kernel, no per-step sort
     int tracer_kernel = 0;         // velocity loop and samples: 0 automatic, forced 1 bricks, 2 global gather, 3 column walk
     int tracer_form = 0;           // the form chosen for this tracer set (0: not yet)
+    int nine_form = 0;             // 9-plane samples before its first loop (0: not chosen)
+    bool nine_sampled = false;     // the set had a 9-plane sample
+    bool looped = false;           // and a velocity loop
     // device buffers (element size es = sizeof(rnumber))
     size_t es = 4;
     size_t ps = 0;                 // complex elements per plane, row pads included (plane_size)

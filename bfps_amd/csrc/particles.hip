@@ -1628,139 +1628,173 @@ int loop_form(bfpsh_ctx* ctx, int form, const void* u, double dt, int order) {
     return BFPSH_OK;
 }
 
+// Bucket the tracers as form `form` needs them.  Bricks and columns need the
+// buckets of every call, the gather a permutation sort_every steps old.
+template <typename T, int NB>
+int sort_form(bfpsh_ctx* ctx, int form) {
+    if constexpr (ColCfg<T, NB>::ok)
+        if (form == FORM_COLUMN) {
+            ColGeom g;
+            col_geom<T, NB>(ctx, g);
+            return sort_cols<T, NB>(ctx, g);
+        }
+    if constexpr (BrickCfg<T, NB>::ok)
+        if (form == FORM_BRICK) return sort_bricks<T, NB>(ctx);
+    return sort_tracers(ctx);
+}
+
+// The fastest of the applicable forms, another than the first only when it is
+// more than 10 % faster (near ties keep the first, so that runs choose alike).
+// With d_out: the 9-plane sample of f, into d_out; else the velocity loop of
+// the highest order with dt = 0 on a copy of the tracer state, f its velocity.
+template <typename T, int NB>
+int time_forms(bfpsh_ctx* ctx, const int* cand, int ncand, const void* f, double* d_out, int* best_form) {
+    static const char* const names[4] = {"auto", "bricks", "global gather", "column walk"};
+    const bool nine = d_out != nullptr, verbose = std::getenv("BFPSH_TRACER_VERBOSE") != nullptr;
+    // the loop's trials move a copy of the positions with a zeroed history; the
+    // copy is refreshed before every launch sequence, so that each one
+    // locates the tracers from the real positions whatever the previous
+    // one left (its dt = 0 move adds 0 x the interpolated values)
+    const size_t pos_bytes = size_t(ctx->np) * 3 * sizeof(double);
+    const size_t rhs_bytes = size_t(ctx->nsteps) * pos_bytes;
+    double *spos = nullptr, *srhs = nullptr;
+    hipEvent_t a = nullptr, b = nullptr;
+    if (!nine) {
+        if (hipMalloc((void**)&spos, pos_bytes) != hipSuccess || hipMalloc((void**)&srhs, rhs_bytes) != hipSuccess) {
+            // no memory for a copy: no trials
+            (void)hipGetLastError();
+            (void)hipFree(spos);
+            *best_form = cand[0];
+            return BFPSH_OK;
+        }
+        HIPCHK(hipMemsetAsync(srhs, 0, rhs_bytes, ctx->stream));
+    }
+    HIPCHK(hipEventCreate(&a));
+    HIPCHK(hipEventCreate(&b));
+    double* const pos = ctx->d_pos;
+    double* const rhs = ctx->d_rhs;
+    const bool prof = ctx->prof, add_head = ctx->add_head;
+    ctx->prof = false;  // the trials stay out of the kernel profile
+    if (!nine) {
+        ctx->d_pos = spos;
+        ctx->d_rhs = srhs;
+    }
+    ctx->add_head = false;
+    auto trial = [&](int c, int planes) -> int {
+        return nine ? sample_form<T, NB>(ctx, c, f, planes, d_out) : loop_form<T, NB>(ctx, c, f, 0.0, ctx->nsteps);
+    };
+    // the state of a step before form c: positions, and for the gather its
+    // permutation (which it renews every sort_every steps)
+    auto fresh = [&](int c) -> int {
+        if (!nine && hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+            return BFPSH_EHIP;
+        ctx->sort_age = c == FORM_GATHER && ctx->sort_every > 1 ? 0 : 1 << 30;
+        return BFPSH_OK;
+    };
+    double tbest = 1e300, tfirst = 0.0;
+    int best = cand[0], r = BFPSH_OK;
+    for (int i = 0; i < ncand && r == BFPSH_OK; i++) {
+        float ms = 0.f;
+        auto timed = [&](int planes) -> int {
+            const int q0 = fresh(cand[i]);
+            if (q0) return q0;
+            if (hipEventRecord(a, ctx->stream) != hipSuccess) return BFPSH_EHIP;
+            const int q = trial(cand[i], planes);
+            if (q) return q;
+            return hipEventRecord(b, ctx->stream) == hipSuccess && hipEventSynchronize(b) == hipSuccess &&
+                           hipEventElapsedTime(&ms, a, b) == hipSuccess
+                       ? BFPSH_OK
+                       : BFPSH_EHIP;
+        };
+        // the form's first buckets allocate and wait, and are the gather's
+        // permutation: outside the timed part
+        if (!nine && hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+            r = BFPSH_EHIP;
+        if (r == BFPSH_OK) r = sort_form<T, NB>(ctx, cand[i]);
+        // warm-up: the first form's may load the code (14 ms), three planes
+        // do; a later form's nine planes that take above 1 ms and longer
+        // than a form timed before are not repeated (2^19 tracers, n = 6,
+        // 256^3: the choice takes 19 instead of 31 ms)
+        if (r == BFPSH_OK) r = timed(nine && i > 0 ? 9 : 3);
+        if (r == BFPSH_OK && !(nine && i > 0 && ms > 1.f && ms > tbest)) r = timed(nine ? 9 : 3);
+        if (i == 0) tfirst = ms;
+        if (r == BFPSH_OK && verbose)
+            std::fprintf(stderr, "bfpsh: tracer form trial (n = %d, %s tracers, %lld of them%s): %s %.3f ms\n", NB,
+                         sizeof(T) == 8 ? "FP64" : "FP32", (long long)ctx->np, nine ? ", 9-plane sample" : "",
+                         names[cand[i]], ms);
+        if (r == BFPSH_OK && ms < tbest) {
+            tbest = ms;
+            best = cand[i];
+        }
+    }
+    if (tbest > 0.9 * tfirst) best = cand[0];
+    if (r == BFPSH_OK && verbose) std::fprintf(stderr, "bfpsh: tracer form chosen: %s\n", names[best]);
+    // the trials' launches are done before the copies are freed
+    if (r == BFPSH_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) r = BFPSH_EHIP;
+    ctx->d_pos = pos;
+    ctx->d_rhs = rhs;
+    ctx->add_head = add_head;
+    ctx->prof = prof;
+    (void)hipEventDestroy(a);
+    (void)hipEventDestroy(b);
+    (void)hipFree(spos);
+    (void)hipFree(srhs);
+    ctx->sort_age = 1 << 30;  // the trials' sorts leave another order behind
+    if (r) return r == BFPSH_EHIP ? fail(ctx, r, "tracer kernel choice: HIP error") : r;
+    *best_form = best;
+    return BFPSH_OK;
+}
+
 // The kernel form of a box's velocity loop and samples: the forced one if it
-// applies; else, once per tracer set, the form whose velocity loop (sort,
-// interpolation, Adams-Bashforth move of the highest order) runs fastest,
-// timed on a copy of the tracer state with dt = 0, when it beats the first
-// applicable one by more than 10 % (plan rigor MEASURE or PATIENT, as the
-// pass autotuner), or the first applicable of column walk, bricks, global
-// gather (ESTIMATE).  When a sample of nine planes comes first, the trials are
-// that sample, into its own output: the walks and bricks stage planes whole,
-// the gather reads lines per tracer and plane, so three planes and a move do
-// not tell which is faster for nine (256^3 FP32, 10^5 tracers, n = 4: the loop
-// is fastest by the gather, the gradient sample by columns, 0.63 ms against
-// 0.87 by bricks and 1.37 by the gather).  One form serves the loop and all
-// samples of a tracer set, so that results do not mix forms.
-// The loop's trials interpolate ctx->ru, or the field f of nc
-// planes about to be sampled when ctx->ru is not allocated yet; with
-// neither (a 1-plane sample first) this call takes the first applicable
-// form and the choice waits for a later call.  The forms sum in different
-// orders: results agree to rounding, not bit for bit.  BFPSH_TRACER_VERBOSE
-// set in the environment prints the trials to stderr.
+// applies; else (plan rigor MEASURE or PATIENT, as the pass autotuner) the
+// fastest velocity loop, timed at the first call of a tracer set; at ESTIMATE
+// the first applicable of column walk, bricks, global gather.  The loop decides
+// whatever the first call is, since it runs every step (128^3 FP64, 10^5
+// tracers, n = 2: 64 us by the gather, 126 by columns, which a 9-plane sample
+// would choose, 271 against 292 us).  A set that is only sampled has no loop to
+// pay for: from the second 9-plane sample before any loop on, these run in the
+// form fastest at that (256^3 FP32, 10^5 tracers, n = 4: 1.40 ms by the loop's
+// gather, 0.61 by columns), until the first loop; from then on one form serves
+// all calls.  The walks and bricks stage planes whole, the gather reads lines
+// per tracer and plane: three planes and a move do not tell which is faster for
+// nine.  The loop's trials interpolate ctx->ru, or the field f of nc planes
+// about to be sampled when ctx->ru is not allocated yet; with neither (a
+// 1-plane sample first) this call takes the first applicable form and the
+// choice waits for a later call.  The forms sum in different orders: results
+// agree to rounding, not bit for bit.  BFPSH_TRACER_VERBOSE set in the
+// environment prints the trials to stderr.
 template <typename T, int NB>
 int tracer_form(bfpsh_ctx* ctx, const void* f, int nc, double* d_out, int* form) {
-    static const char* const names[4] = {"auto", "bricks", "global gather", "column walk"};
     if (ctx->tracer_kernel != FORM_AUTO && form_ok<T, NB>(ctx, ctx->tracer_kernel)) {
         *form = ctx->tracer_kernel;
-        return BFPSH_OK;
-    }
-    if (ctx->tracer_form != FORM_AUTO) {
-        *form = ctx->tracer_form;
         return BFPSH_OK;
     }
     int cand[3], ncand = 0;
     for (int c : {int(FORM_COLUMN), int(FORM_BRICK), int(FORM_GATHER)})
         if (form_ok<T, NB>(ctx, c)) cand[ncand++] = c;
-    int best = cand[0];
-    const bool nine = nc == 9;
-    const void* u = ctx->ru && !nine ? ctx->ru : (nc >= 3 ? f : nullptr);
-    if (ncand > 1 && ctx->plan_rigor != BFPSH_ESTIMATE && ctx->tracer_kernel == FORM_AUTO && !u) {
-        *form = best;
-        return BFPSH_OK;
+    const bool trials = ncand > 1 && ctx->plan_rigor != BFPSH_ESTIMATE && ctx->tracer_kernel == FORM_AUTO;
+    if (ctx->tracer_form == FORM_AUTO) {
+        int best = cand[0];
+        if (trials) {
+            const void* u = ctx->ru ? ctx->ru : (nc >= 3 ? f : nullptr);
+            if (!u) {
+                *form = best;
+                return BFPSH_OK;
+            }
+            int r = time_forms<T, NB>(ctx, cand, ncand, u, nullptr, &best);
+            if (r) return r;
+        }
+        ctx->tracer_form = best;
     }
-    if (ncand > 1 && ctx->plan_rigor != BFPSH_ESTIMATE && ctx->tracer_kernel == FORM_AUTO) {
-        // the trials move a copy of the positions with a zeroed history; the
-        // copy is refreshed before every launch sequence, so that each one
-        // locates the tracers from the real positions whatever the previous
-        // one left (its dt = 0 move adds 0 x the interpolated values)
-        const size_t pos_bytes = size_t(ctx->np) * 3 * sizeof(double);
-        const size_t rhs_bytes = size_t(ctx->nsteps) * pos_bytes;
-        double *spos = nullptr, *srhs = nullptr;
-        hipEvent_t a = nullptr, b = nullptr;
-        if (!nine) {
-            HIPCHK(hipMalloc((void**)&spos, pos_bytes));
-            if (hipMalloc((void**)&srhs, rhs_bytes) != hipSuccess) {
-                (void)hipFree(spos);
-                return fail(ctx, BFPSH_EHIP, "tracer kernel choice: device memory for the trial state");
-            }
-            HIPCHK(hipMemsetAsync(srhs, 0, rhs_bytes, ctx->stream));
+    *form = ctx->tracer_form;
+    if (nc == 9 && trials && !ctx->looped) {
+        if (ctx->nine_form == FORM_AUTO && ctx->nine_sampled) {
+            int r = time_forms<T, NB>(ctx, cand, ncand, f, d_out, &ctx->nine_form);
+            if (r) return r;
         }
-        HIPCHK(hipEventCreate(&a));
-        HIPCHK(hipEventCreate(&b));
-        double* const pos = ctx->d_pos;
-        double* const rhs = ctx->d_rhs;
-        const bool prof = ctx->prof, add_head = ctx->add_head;
-        ctx->prof = false;  // the trials stay out of the kernel profile
-        if (!nine) {
-            ctx->d_pos = spos;
-            ctx->d_rhs = srhs;
-        }
-        ctx->add_head = false;
-        auto trial = [&](int c, int planes) -> int {
-            return nine ? sample_form<T, NB>(ctx, c, u, planes, d_out) : loop_form<T, NB>(ctx, c, u, 0.0, ctx->nsteps);
-        };
-        auto fresh = [&]() -> int {
-            if (!nine && hipMemcpyAsync(spos, pos, pos_bytes, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
-                return BFPSH_EHIP;
-            ctx->sort_age = 1 << 30;  // bricks and columns sort, as in a step
-            return BFPSH_OK;
-        };
-        double tbest = 1e300, tfirst = 0.0;
-        int r = BFPSH_OK;
-        for (int i = 0; i < ncand && r == BFPSH_OK; i++) {
-            float ms = 0.f;
-            auto timed = [&](int planes) -> int {
-                if (hipEventRecord(a, ctx->stream) != hipSuccess) return BFPSH_EHIP;
-                const int q = trial(cand[i], planes);
-                if (q) return q;
-                return hipEventRecord(b, ctx->stream) == hipSuccess && hipEventSynchronize(b) == hipSuccess &&
-                               hipEventElapsedTime(&ms, a, b) == hipSuccess
-                           ? BFPSH_OK
-                           : BFPSH_EHIP;
-            };
-            r = fresh();
-            // warm-up: the first form's may load the code (14 ms), three planes
-            // do; a later form's nine planes that take above 1 ms and longer
-            // than a form timed before are not repeated (2^19 tracers, n = 6,
-            // 256^3: first gradient sample 30.7 -> 19.4 ms)
-            if (r == BFPSH_OK) r = timed(nine && i > 0 ? 9 : 3);
-            if (r == BFPSH_OK && !(nine && i > 0 && ms > 1.f && ms > tbest)) {
-                r = fresh();
-                // (the gather renews its permutation every sort_every steps:
-                // it is timed on the one of its warm-up)
-                if (cand[i] == FORM_GATHER && ctx->sort_every > 1) ctx->sort_age = 0;
-                if (r == BFPSH_OK) r = timed(nine ? 9 : 3);
-            }
-            if (i == 0) tfirst = ms;
-            if (r == BFPSH_OK && std::getenv("BFPSH_TRACER_VERBOSE"))
-                std::fprintf(stderr, "bfpsh: tracer form trial (n = %d, %s tracers, %lld of them%s): %s %.3f ms\n",
-                             NB, sizeof(T) == 8 ? "FP64" : "FP32", (long long)ctx->np,
-                             nine ? ", 9-plane sample" : "", names[cand[i]], ms);
-            if (r == BFPSH_OK && ms < tbest) {
-                tbest = ms;
-                best = cand[i];
-            }
-        }
-        // another form only when clearly faster: near ties keep the
-        // first applicable form, so that runs choose alike
-        if (tbest > 0.9 * tfirst) best = cand[0];
-        if (r == BFPSH_OK && std::getenv("BFPSH_TRACER_VERBOSE"))
-            std::fprintf(stderr, "bfpsh: tracer form chosen: %s\n", names[best]);
-        // the trials' launches are done before the copies are freed
-        if (r == BFPSH_OK && hipStreamSynchronize(ctx->stream) != hipSuccess) r = BFPSH_EHIP;
-        ctx->d_pos = pos;
-        ctx->d_rhs = rhs;
-        ctx->add_head = add_head;
-        ctx->prof = prof;
-        (void)hipEventDestroy(a);
-        (void)hipEventDestroy(b);
-        (void)hipFree(spos);
-        (void)hipFree(srhs);
-        if (r) return r == BFPSH_EHIP ? fail(ctx, r, "tracer kernel choice: HIP error") : r;
-        ctx->sort_age = 1 << 30;  // the trials' sorts leave another order behind
+        if (ctx->nine_form != FORM_AUTO) *form = ctx->nine_form;
+        ctx->nine_sampled = true;
     }
-    ctx->tracer_form = best;
-    *form = best;
     return BFPSH_OK;
 }
 
@@ -1969,6 +2003,7 @@ int bfpsh_part_ens_launch(PartBatch* pb, int ngroups) {
 void bfpsh_part_ens_advanced(const std::vector<bfpsh_ctx*>& boxes, PartBatch* pb, int ngroups) {
     // the host's view of every box follows the device's k_tracer_dyn_advance
     for (bfpsh_ctx* c : boxes) {
+        c->looped = true;
         c->sort_age += 1;
         c->step_idx += 1;
         c->head = (c->head + c->nsteps - 1) % c->nsteps;
@@ -2018,6 +2053,7 @@ int bfpsh_part_loop(bfpsh_ctx* ctx, double dt) {
     const int order = std::min(ctx->step_idx, ctx->nsteps);
     int r = ctx->prec == BFPSH_FP32 ? loop_t<float>(ctx, dt, order) : loop_t<double>(ctx, dt, order);
     if (r) return r;
+    ctx->looped = true;
     ctx->sort_age += 1;
     ctx->step_idx += 1;
     ctx->head = (ctx->head + ctx->nsteps - 1) % ctx->nsteps;

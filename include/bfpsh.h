@@ -75,11 +75,12 @@ int bfpsh_create(bfpsh_ctx** out, int nx, int ny, int nz, double dkx, double dky
  * the first tracer loop or sample of a tracer set also times the velocity
  * loop of each applicable tracer kernel form (column walk, bricks, global
  * gather) on a device copy of the tracer state, which it allocates for the
- * time it runs (or the 9-plane sample itself, where that comes first), and
- * keeps the fastest when it is more than 10 % faster
- * than the first applicable one (BFPSH_TRACER_KERNEL=column|brick|gather
- * in the environment forces a form, BFPSH_TRACER_VERBOSE prints the
- * trials). */
+ * time it runs, and keeps the fastest when it is more than 10 % faster than
+ * the first applicable one (which it takes without memory for the copy).
+ * The second 9-plane sample of a set that had no loop yet times that sample
+ * by each form likewise, for such samples until the first loop
+ * (BFPSH_TRACER_KERNEL=column|brick|gather in the environment forces a form,
+ * BFPSH_TRACER_VERBOSE prints the trials). */
 enum { BFPSH_ESTIMATE = 0, BFPSH_MEASURE = 1, BFPSH_PATIENT = 2 };
 /* strided pass kinds: inverse and forward transforms along kz (z) and ky
  * (y), the vorticity step's fused first pass (Biot-Savart + inverse y) and
