@@ -13,7 +13,6 @@
 // overlap.
 #include <condition_variable>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "ctx.hpp"
@@ -111,8 +110,11 @@ int run_chunks(bfpsh_ctx* ctx, size_t nchunks, W&& work) {
     for (int t = 1; t < nt; t++) {
         try {
             th[t] = std::thread(body, t);
-        } catch (const std::system_error&) {
-            here[t] = true;  // no thread to be had: this one takes its chunks
+        } catch (...) {
+            // no thread (or no memory for one) to be had: this one takes its
+            // chunks.  Nothing may pass here: threads already started use
+            // this frame
+            here[t] = true;
         }
     }
     body(0);
