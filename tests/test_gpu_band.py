@@ -4,13 +4,15 @@ kx = 0 plane factor that stands in for the symmetrized velocity, and both
 forms of the integrating factor, against the CPU oracle.
 
 Tolerance: relative L2 1e-11 after a few FP64 steps, that of the other FP64
-step tests (rounding of 27 transforms a step, about 1e-15 each).
+step tests (rounding of 27 transforms a step, about 1e-15 each), and 1e-6 in
+FP32 (about 1e-7 each).
 """
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-11
+TOL32 = 1e-6
 
 
 def rel(a, b):
@@ -63,6 +65,75 @@ def test_step(oracle, n, dealias, projected, dk, nu):
     e = rel(fs.cvorticity, o.get_cfield("vorticity"))
     print("  rel", e, flush=True)
     assert e < TOL
+
+
+@pytest.mark.parametrize("n, dealias, projected", [
+    (32, "TWO_THIRDS", True), (32, "SMOOTH", False),     # one launch a stage over the (z, x) slab of a y
+    (64, "TWO_THIRDS", True), (64, "TWO_THIRDS", False), (64, "SMOOTH", False),  # the same, FP32 only
+    (48, "TWO_THIRDS", False),
+    (128, "TWO_THIRDS", True), (128, "SMOOTH", False),   # x pass in registers, FP32 only
+])
+def test_step_single(oracle, n, dealias, projected):
+    import bfps_amd as B
+    w0 = spectrum(n, n + 2).astype(np.complex64)
+    print("case: band fp32 n=%d %s projected=%s" % (n, dealias, projected), flush=True)
+    fs = B.vorticity_equation("t", n, precision="single", dealias=dealias)
+    fs.nu, fs.famplitude, fs.forcing_type = 0.02, 0.3, "linear"
+    o = oracle.Solver(n, precision="double", dealias=dealias)
+    o.set_physics(0.02, "linear", 0.3, 2.0, 4.0)
+    o.set_cfield("vorticity", w0.astype(np.complex128))
+    if projected:
+        fs.io_checkpoint(read=True, data=w0)
+        o.io_projection()
+    else:
+        fs.cvorticity = w0
+    for _ in range(2):
+        fs.step(0.005)
+        o.step(0.005)
+    e = rel(fs.cvorticity, o.get_cfield("vorticity"))
+    print("  rel", e, flush=True)
+    assert e < TOL32
+
+
+@pytest.mark.parametrize("precision, dealias, projected", [
+    ("single", "SMOOTH", True), ("single", "TWO_THIRDS", True), ("single", "SMOOTH", False),
+    ("double", "TWO_THIRDS", True)])
+def test_every_band_pass_shape(precision, dealias, projected):
+    """Every shape of the step's z passes, persistent ones among them, by a
+    step at 256^3 from a field that fills the sphere (and, unprojected, what
+    lies beyond it) evenly: as the built-in shapes, which the steps above check,
+    to rounding."""
+    import bfps_amd as B
+    n = 256
+    print("case: band pass shapes %s %s projected=%s" % (precision, dealias, projected), flush=True)
+    fs = B.vorticity_equation("t", n, precision=precision, dealias=dealias, plan_rigor="FFTW_ESTIMATE")
+    fs.nu, fs.forcing_type = 0.0005, "none"
+    rng = np.random.default_rng(n)
+    real = np.float32 if precision == "single" else np.float64
+    w0 = rng.standard_normal((n, n, n // 2 + 1, 6), dtype=real).view(fs.cdtype)
+    w0 *= 0.01  # dt k u is about a quarter: the nonlinear term is a good part of the step
+    w0[:, :, n // 2] = 0
+
+    def step(index):
+        for kind in ("z_inv", "z_fwd"):
+            fs.set_pass_shape(kind, index)
+        if projected:
+            fs.io_checkpoint(read=True, data=w0)
+        else:
+            fs.cvorticity = w0
+        start = fs.cvorticity if index == 0 else None
+        fs.step(0.005)
+        return start, fs.cvorticity
+
+    start, want = step(0)
+    assert rel(want, start) > 0.05
+    shapes = fs.pass_shapes()["z_inv"][3]
+    assert shapes > 8
+    for index in range(1, shapes):
+        e = rel(step(index)[1], want)
+        print("  shape %d %s rel %.3e" % (index, fs.pass_shapes()["z_inv"][:2] + fs.pass_shapes()["z_inv"][4:], e), flush=True)
+        assert e < (TOL32 if precision == "single" else TOL)
+    fs.close()
 
 
 @pytest.mark.parametrize("n, dealias, dk", [
