@@ -189,6 +189,7 @@ struct Impl {
             for (int i = 0; i < rounds * sh.n && rc == BFPSH_OK; i++) {
                 const int v = i % sh.n;
                 const CT* tw = (const CT*)ctx->tw;
+                const int planes = kind == BFPSH_PASS_Z_INV ? 6 : 3;  // that it reads
                 // one launch of shape v: a plain pass over the planes of a step
                 // (one plane would stay in the last-level cache, where other
                 // shapes win), the z passes within the band as the step runs
@@ -208,7 +209,6 @@ struct Impl {
                                     geom(ctx), sp);
                     } else {
                         const bool z = kind == BFPSH_PASS_Z_INV || kind == BFPSH_PASS_Z_FWD;
-                        const int planes = kind == BFPSH_PASS_Z_INV ? 6 : 3;
                         pass_fn(kind, v)(ctx->stream, (CT*)ctx->work, pass_estride(kind), pass_ostride(kind), tw, planes, 0,
                                          1, z ? band(ctx) : nullptr);
                     }
@@ -217,8 +217,9 @@ struct Impl {
                 // grow with each transform, and zeros move and compute at
                 // other speeds (512^3 FP32 forward z pass on zeros: the
                 // slowest of four candidates, 0.675 against 0.58 ms, won)
-                k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>((CT*)ctx->work, 6 * ctx->ps);
-                if (fused) k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>(scratch, 3 * ctx->ps);
+                if (kind != BFPSH_PASS_BS)
+                    k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>((CT*)ctx->work, planes * ctx->ps);
+                if (fused) k_fill_pattern<T><<<2048, 256, 0, ctx->stream>>>(scratch, planes * ctx->ps);
                 run();  // warm-up
                 (void)hipEventRecord(a, ctx->stream);
                 for (int r = 0; r < reps; r++) run();
