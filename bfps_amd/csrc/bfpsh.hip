@@ -1047,7 +1047,9 @@ static int ensemble_capture(bfpsh_ensemble* e, bool with_ru, int ngroups) {
         d.v0 = b0->v0;
         d.v1 = b0->v1;
         d.v2 = b0->v2;
-        d.w = b0->work;
+        // the work planes of the slab, not b0->work: a gradient moves a box's
+        // own to a larger allocation outside, bstride from which lies nothing
+        d.w = (char*)c.slab + 9 * plane_size(c.n) * 2 * b0->es;
         d.ru = with_ru ? b0->ru : nullptr;
         rc = ops_for(b0)->batch_step(b0, d);
         if (rc) {

@@ -148,3 +148,31 @@ def test_ensemble_full_manifest(B, oracle):
     sep.close()
     assert gsi == osi == nsteps + 1
     assert e < 3e-6 and ep < 1e-7 and er < 1e-5
+
+
+@pytest.mark.parametrize("boxes_with_gradient", [(0,), (1, 2)])
+def test_gradient_of_a_box_between_steps(B, boxes_with_gradient):
+    """A gradient gives a box a larger work buffer outside the class's slab.
+    The steps go on in the slab, whichever box it was, before the first step
+    and before the graph is captured anew (an unprojected field put): bit for
+    bit as without the gradients."""
+    from bfps_amd import ic
+    n, dt = 32, 0.01
+
+    def run(gradients):
+        ens = B.ensemble([n, n, n], precision="double")
+        for i, b in enumerate(ens.boxes):
+            b.nu, b.forcing_type = 0.02, "none"
+            b.io_checkpoint(read=True, data=ic.solenoidal_vorticity(n, seed=7 + i, k0=4.0, dtype=b.cdtype))
+        for put in (False, True):
+            if put:
+                ens.boxes[1].cvorticity = ic.solenoidal_vorticity(n, seed=17, k0=4.0, dtype=ens.boxes[1].cdtype)
+            for i in gradients:
+                ens.boxes[i].gradient_rspace()
+            for _ in range(2):
+                ens.step(dt, with_particles=False)
+        return [b.cvorticity for b in ens.boxes]
+
+    print("case: ensemble, gradients of boxes %s" % (boxes_with_gradient,), flush=True)
+    for a, b in zip(run(boxes_with_gradient), run(())):
+        assert np.array_equal(a, b)
