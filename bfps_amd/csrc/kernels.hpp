@@ -1086,33 +1086,36 @@ k_rows_r2c(const T* data, C2<T>* out, const C2<T>* __restrict__ tw) {
 }
 
 // ------------------------------------------------------------ integrating factor
-// exp(x + y) as `one` + a b + (a lb + la b) from a part a, la of x and b, lb
-// of y, which depend on fewer indexes than their sum.  While the factors stay
-// above exp(-1/2) (`slow`, uniform; one = 1), a = exp(x) - 1 and la = 1: 1 +
-// (a + b + a b), whose error is that of its last rounding, like an
-// exponential's own.  Beyond (one = 0), that sum would cancel, and a product
-// of two rounded exponentials has 1.3 times an exponential's error: there
-// exp(x) = a + la, a its rounded value and la the rest, from x = m ln 2 + r,
-// |r| <= ln 2 / 2 (argument reduction of Cody and Waite) and exp(r) - 1.
+// exp(x + y) from a part a, ra of x and b, rb of y, which depend on fewer
+// indexes than their sum.  While the factors stay above exp(-1/2) (`slow`,
+// uniform; one = 1), a = exp(x) - 1, ra = 0 and the factor is 1 + (a + b + a b),
+// whose error is that of its last rounding, like an exponential's own.  Beyond
+// (one = 0), that sum would cancel, and a product of two rounded exponentials
+// has 1.3 times an exponential's error: there exp(x) = a (1 + ra), a its rounded
+// value and ra the rest, from x = m ln 2 + r, |r| <= ln 2 / 2 (argument
+// reduction of Cody and Waite) and exp(r) - 1, and the factor a b + a b (ra +
+// rb).  The rest is relative, so that it neither over- nor underflows in 32 bits.
 // FP64 decay at 64^3 over 64 steps, mean error of a mode at nu dt kM^2 = 1.4 /
 // 3: 7.8e-15 / 1.00e-14; by products 1.02e-14 / 1.29e-14; with one rounded
 // exponential a factor 8.3e-15 / 9.7e-15.
 BFPSH_DEV double if_part(double x, bool slow, float& rest) {
     double q = 0.0;
     if (!slow) {
-        q = rint(fmin(fmax(x * 0x1.71547652b82fep+0, -8000.0), 8000.0));  // x / ln 2
+        q = rint(fmin(fmax(x * 0x1.71547652b82fep+0, -1e9), 1e9));  // x / ln 2
         // (ln 2 and what its rounding leaves)
         x = fma(-q, 0x1.abc9e3b39803fp-56, fma(-q, 0x1.62e42fefa39efp-1, x));
     }
     const double e = expm1(x);
-    rest = 1.0f;
+    rest = 0.0f;
     if (slow) return e;
     const double h = 1.0 + e;
-    rest = float(ldexp(e - (h - 1.0), int(q)));
+    if (h > 0.0) rest = float((e - (h - 1.0)) / h);
     return ldexp(h, int(q));
 }
-BFPSH_DEV double if_of(double a, double b, float la, float lb, double one) {
-    return one + fma(a, b, fma(a, double(lb), double(la) * b));
+// `one` plus the absolute rest of a part: 1 if slow
+BFPSH_DEV double if_rest(double a, float ra, double one) { return fma(double(ra), a, one); }
+BFPSH_DEV double if_of(double a, double la, double b, double lb, double one) {
+    return one + fma(a, b, fma(a, lb, la * b));
 }
 
 // ------------------------------------------------------------ last forward pass + update
@@ -1188,6 +1191,7 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
     float rxz, rxz1 = 0.f;
     const double ifxz = if_part(-nud * (kx * kx + kzv * kzv), slow, rxz);
     const double ifxz1 = STAGE == 2 ? if_part(nud * (kx * kx + kzv * kzv), slow, rxz1) : 0.0;
+    const double lxz = if_rest(ifxz, rxz, one), lxz1 = if_rest(ifxz1, rxz1, one);
     __syncthreads();
     // one component after the other; an opaque group index and table offset
     // per component, so that twiddles and LDS addresses are not held across,
@@ -1275,13 +1279,14 @@ k_y_update(C2<T>* w, const C2<T>* v0, const C2<T>* vp, C2<T>* dst, const C2<T>* 
             const double ik2 = k2 > 0 ? 1.0 / k2 : 0.0;  // one division, then products
             if (k2 > 0) divfree<T>(cu, kx, kyv, kzv, ik2);
             else cu[0] = cu[1] = cu[2] = mk<T>(T(0), T(0));
-            const double f0 = if_of(ifxz, ify[0][ky], rxz, ifr[0][ky], one);
+            const double f0 = if_of(ifxz, lxz, ify[0][ky], if_rest(ify[0][ky], ifr[0][ky], one), one);
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 if constexpr (STAGE == 1) {
                     nv[c] = mk<T>(T((w0[c].x + dt * cu[c].x) * f0), T((w0[c].y + dt * cu[c].y) * f0));
                 } else if constexpr (STAGE == 2) {
-                    const double f1 = if_of(ifxz1, ify[STAGE - 1][ky], rxz1, ifr[STAGE - 1][ky], one);
+                    const double b1 = ify[STAGE - 1][ky];
+                    const double f1 = if_of(ifxz1, lxz1, b1, if_rest(b1, ifr[STAGE - 1][ky], one), one);
                     nv[c] = mk<T>(T((3 * w0[c].x * f0 + (w1[c].x + dt * cu[c].x) * f1) * 0.25),
                                   T((3 * w0[c].y * f0 + (w1[c].y + dt * cu[c].y) * f1) * 0.25));
                 } else {

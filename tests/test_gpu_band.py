@@ -215,6 +215,29 @@ def test_strong_damping(x):
     assert e < 1.15 * one
 
 
+def test_inverse_factors_beyond_32_bits(oracle):
+    """One step whose last modes are damped by exp(-260): the second stage's
+    inverse factors reach exp(130), beyond a 32-bit number's range.  The field
+    is so small (1e-120) that they do not raise the nonlinear term to it."""
+    import bfps_amd as B
+    n, dt = 32, 0.005
+    nu = 260 / (dt * (n // 2 - 1) ** 2)
+    print("case: inverse factors up to exp(130)", flush=True)
+    w0 = spectrum(n, 3) * 1e-120
+    fs = B.vorticity_equation("t", n, precision="double")
+    fs.nu, fs.forcing_type = nu, "none"
+    fs.io_checkpoint(read=True, data=w0)
+    fs.step(dt)
+    o = oracle.Solver(n, precision="double")
+    o.set_physics(nu, "none", 0.0, 2.0, 4.0)
+    o.set_cfield("vorticity", w0)
+    o.io_projection()
+    o.step(dt)
+    e = rel(fs.cvorticity, o.get_cfield("vorticity"))
+    print("  rel", e, flush=True)
+    assert e < TOL
+
+
 def test_put_switches_the_table(oracle):
     """An unprojected put, then a projection, then steps: each form in turn,
     and the same in a box of an ensemble beside a projected one."""
