@@ -1714,7 +1714,7 @@ int time_forms(bfpsh_ctx* ctx, const int* cand, int ncand, const void* f, double
         // warm-up: the first form's may load the code (14 ms), three planes
         // do; a later form's nine planes that take above 1 ms and longer
         // than a form timed before are not repeated (2^19 tracers, n = 6,
-        // 256^3: the choice takes 19 instead of 31 ms)
+        // 256^3: the trials take 13 ms, bricks and gather again another 9)
         if (r == BFPSH_OK) r = timed(nine && i > 0 ? 9 : 3);
         if (r == BFPSH_OK && !(nine && i > 0 && ms > 1.f && ms > tbest)) r = timed(nine ? 9 : 3);
         if (i == 0) tfirst = ms;
